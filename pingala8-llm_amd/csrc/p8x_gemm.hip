@@ -26,13 +26,9 @@
 #include "p8x_internal.h"
 #include "p8x_act.h"
 #include "p8x_lane.h"
+#include "p8x_mm.h"
 
 namespace p8x {
-
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef _Float16 half8v __attribute__((ext_vector_type(8)));
-typedef float float16v __attribute__((ext_vector_type(16)));
-
 
 // ------------------------------------------------------------------------------------------------ pass 1
 // x' = FWHT(x ic) / 16 per 256-block, fp16. Lane holds 4 consecutive elements; butterflies h = 1, 2 in the
@@ -45,28 +41,8 @@ __global__ __launch_bounds__(64 * kMmActWaves) void k_mm_act(const XT *__restric
     const int lane = threadIdx.x & 63, b = kMmActWaves * (int)blockIdx.x + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = blockIdx.y;
     if (256 * b >= K) return;
-    const XT *xp = x + (size_t)n * ldx + 256 * b + 4 * lane;
-    const float4 cv = *reinterpret_cast<const float4 *>(ic + 256 * b + 4 * lane);
-    float v[4];
-    if constexpr (sizeof(XT) == 4) {
-        v[0] = xp[0]; v[1] = xp[1]; v[2] = xp[2]; v[3] = xp[3];
-    } else {
-        const uint2 raw = *reinterpret_cast<const uint2 *>(xp);
-        v[0] = bf16_to_float((uint16_t)raw.x); v[1] = bf16_to_float((uint16_t)(raw.x >> 16));
-        v[2] = bf16_to_float((uint16_t)raw.y); v[3] = bf16_to_float((uint16_t)(raw.y >> 16));
-    }
-    v[0] *= cv.x; v[1] *= cv.y; v[2] *= cv.z; v[3] *= cv.w;
-    { const float a0 = v[0], b0 = v[1], a1 = v[2], b1 = v[3]; v[0] = a0 + b0; v[1] = a0 - b0; v[2] = a1 + b1; v[3] = a1 - b1; }
-    { const float a0 = v[0], b0 = v[2], a1 = v[1], b1 = v[3]; v[0] = a0 + b0; v[2] = a0 - b0; v[1] = a1 + b1; v[3] = a1 - b1; }
-    fwht_lane_stage<1>(v, lane);
-    fwht_lane_stage<2>(v, lane);
-    fwht_lane_stage<4>(v, lane);
-    fwht_lane_stage<8>(v, lane);
-    fwht_lane_stage<16>(v, lane);
-    fwht_lane_stage<32>(v, lane);
     half2v lo, hi;
-    lo.x = (_Float16)(v[0] * 0.0625f); lo.y = (_Float16)(v[1] * 0.0625f);
-    hi.x = (_Float16)(v[2] * 0.0625f); hi.y = (_Float16)(v[3] * 0.0625f);
+    rotate_f16(x + (size_t)n * ldx + 256 * b, ic + 256 * b, lane, lo, hi);
     uint2 out;
     out.x = __builtin_bit_cast(uint32_t, lo);
     out.y = __builtin_bit_cast(uint32_t, hi);
@@ -88,41 +64,6 @@ struct MmJob {
 #endif
 };
 
-// offset-binary int8x4 (v + 128 per byte) -> two fp16 pairs holding 1152 + v exactly
-__device__ __forceinline__ half2v ob_lo(uint32_t w) { return __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, w, 0x04010400u)); }
-__device__ __forceinline__ half2v ob_hi(uint32_t w) { return __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, w, 0x04030402u)); }
-
-// LDS words of chunk t, all stages (table bytes are A[f] + h c offset by 128)
-template <int C, int NWMAX>
-__device__ __forceinline__ void lookup_chunk(const AnySlice<NWMAX> &ls, const uint32_t *tab, int t, uint32_t hq, uint32_t (&w)[3]) {
-    constexpr int NST = nstage_of(C);
-    w[0] = lds_word(tab, ls.template addr<C, 0>(t, hq));
-    if constexpr (NST > 1) w[1] = lds_word(tab, ls.template addr<C, 1>(t, hq));
-    if constexpr (NST > 2) w[2] = lds_word(tab, ls.template addr<C, 2>(t, hq));
-}
-
-// table words of one chunk -> 4 fp16 weights v S (v exact in fp16, |v| <= 1596; one rounding for the product)
-template <int C>
-__device__ __forceinline__ void weights_chunk(const uint32_t (&w)[3], half2v s2, half2v &lo, half2v &hi) {
-    constexpr int NST = nstage_of(C), SH1 = sh1_of(C), SH2 = sh2_of(C);
-    const half2v bias = {(_Float16)-1152.f, (_Float16)-1152.f};
-    half2v vl = ob_lo(w[0]) + bias, vh = ob_hi(w[0]) + bias;
-    if constexpr (NST > 1) {
-        const half2v m1 = {(_Float16)(float)(1 << SH1), (_Float16)(float)(1 << SH1)};
-        const half2v m2 = {(_Float16)(float)(1 << SH2), (_Float16)(float)(1 << SH2)};
-        half2v al = (ob_lo(w[1]) + bias) * m2, ah = (ob_hi(w[1]) + bias) * m2;
-        if constexpr (NST > 2) { al += ob_lo(w[2]) + bias; ah += ob_hi(w[2]) + bias; }
-        vl = vl * m1 + al;   // integers below 2048: exact in fp16
-        vh = vh * m1 + ah;
-    }
-    lo = vl * s2;
-    hi = vh * s2;
-}
-
-// classes decoded by an instantiation: the tensor's class set (class 0 decodes as zeros in all of them)
-constexpr int kMmCmC3 = 1 << 3, kMmCmAll = 0xFE;
-constexpr int kMmMain = 3;   // the class with a branch-free path in every instantiation (the 2-bit bulk)
-__host__ __device__ constexpr int mm_nwmax(int cm) { return cm == kMmCmC3 ? 8 : 24; }
 // Tile shape (one wave per SIMD, four per workgroup): a wave holds NTI x NTJ MFMA tiles of 32 tokens x 32 weight
 // rows, 16 NTI NTJ fp32 accumulators per lane, for all the workgroup's tokens and its own 32 NTJ rows. Each decoded
 // B operand feeds NTI MFMAs, so the decode work per MFMA falls as 1 / NTI: the class-3 kernel takes 8 x 2 (256
@@ -627,6 +568,7 @@ static int grow(void **p, size_t *have, size_t need, const char *what) {
 }
 
 struct MmPlan {
+    int rg;    // 32-token tiles of the row-group GEMM (p8x_mm_rg.hip), which writes y itself; 0: k_mm, below
     int nti;   // token tiles per wave: the workgroup tile is 256 rows x 32 nti tokens
     int tiles_m, tiles_n, nsplit, kper;
 };
@@ -634,7 +576,7 @@ struct MmPlan {
 // One workgroup per CU. Estimated time = rounds of workgroups x (the measured prologue + blocks per workgroup x the
 // measured time of one K block of a workgroup tile of the shape) + when planes are used (K split, or rows to
 // un-permute) their traffic (written by k_mm, read by k_mm_finish at ~5 TB/s) and k_mm_finish's launch.
-static bool mm_only_c3(const p8x_tensor *t) {
+bool mm_only_c3(const p8x_tensor *t) {
     for (int c = 1; c < 8; ++c) if (c != 3 && t->class_tiles[c]) return false;
     return true;
 }
@@ -647,7 +589,8 @@ static MmPlan mm_plan(const p8x_tensor *t, int N) {
     // plan (and returns the same bits) as p8x_mul_mat wherever it runs at all
     const size_t xb = ((size_t)N * t->K * sizeof(_Float16) + 255) & ~(size_t)255;
     const size_t cap = xb < (size_t)P8X_NOALLOC_SCRATCH_BYTES ? (size_t)P8X_NOALLOC_SCRATCH_BYTES - xb : 0;
-    MmPlan best{4, 0, 0, 1, t->nb};
+    MmPlan best{mm_rg_tiles(t, N), 4, 0, 0, 1, t->nb};
+    if (best.rg) return best;
     double best_cost = -1.0;
     for (int nti = 8; nti >= 4; nti -= 4) {
         if (nti == 8 && !c3) continue;   // the every-class decode needs the registers of the 4 x 2 shape
@@ -661,31 +604,33 @@ static MmPlan mm_plan(const p8x_tensor *t, int N) {
             if (nsr > 1 && (size_t)nsr * N * t->rows * 4 > cap) continue;
             const bool planes = nsr > 1 || !t->prm_identity;
             const double cost = (double)((base * nsr + slots - 1) / slots) * (pro_us + kper * block_us) + (planes ? nsr * plane_us + finish_us : 0.0);
-            if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = MmPlan{nti, tiles_m, tiles_n, nsr, kper}; }
+            if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = MmPlan{0, nti, tiles_m, tiles_n, nsr, kper}; }
         }
     }
     return best;
 }
 
-int reserve_mul_mat(const p8x_tensor *t, int n_max) {
-    p8x_tensor *tw = const_cast<p8x_tensor *>(t);
-    int rc;
-    if ((rc = grow((void **)&tw->wx16, &tw->wx16_elems, (size_t)n_max * t->K * sizeof(_Float16), "p8x_mul_mat_reserve: activation workspace"))) return rc;
-    size_t planes = 0;   // the largest plane need over every N <= n_max (the split count depends on N)
-    for (int n = 1; n <= n_max; ++n) {
-        const MmPlan p = mm_plan(t, n);
-        if (!(p.nsplit == 1 && t->prm_identity)) planes = std::max(planes, (size_t)p.nsplit * n * t->rows * 4);
-    }
-    if (planes && (rc = grow((void **)&tw->wmm, &tw->wmm_bytes, planes, "p8x_mul_mat_reserve: output planes"))) return rc;
-    return P8X_OK;
-}
-
-// workspace bytes of one prompt GEMM call: rotated fp16 activations [N][K], and (K split or rows to un-permute) the
-// sorted-row output planes [nsplit][N][rows] f32
+// workspace bytes of one prompt GEMM call: rotated fp16 activations ([N][K], or whole 32-token tiles), and (k_mm with a
+// K split or rows to un-permute) the sorted-row output planes [nsplit][N][rows] f32
 static void mm_workspace(const p8x_tensor *t, int N, size_t *x_bytes, size_t *plane_bytes) {
     const MmPlan p = mm_plan(t, N);
-    *x_bytes = (size_t)N * t->K * sizeof(_Float16);
-    *plane_bytes = p.nsplit == 1 && t->prm_identity ? 0 : (size_t)p.nsplit * N * t->rows * 4;
+    *x_bytes = p.rg ? mm_rg_x_bytes(t, p.rg) : (size_t)N * t->K * sizeof(_Float16);
+    *plane_bytes = p.rg || (p.nsplit == 1 && t->prm_identity) ? 0 : (size_t)p.nsplit * N * t->rows * 4;
+}
+
+int reserve_mul_mat(const p8x_tensor *t, int n_max) {
+    p8x_tensor *tw = const_cast<p8x_tensor *>(t);
+    size_t xb = 0, planes = 0;   // the largest needs over every N <= n_max (the split count depends on N)
+    for (int n = 1; n <= n_max; ++n) {
+        size_t x1, p1;
+        mm_workspace(t, n, &x1, &p1);
+        xb = std::max(xb, x1);
+        planes = std::max(planes, p1);
+    }
+    int rc;
+    if ((rc = grow((void **)&tw->wx16, &tw->wx16_elems, xb, "p8x_mul_mat_reserve: activation workspace"))) return rc;
+    if (planes && (rc = grow((void **)&tw->wmm, &tw->wmm_bytes, planes, "p8x_mul_mat_reserve: output planes"))) return rc;
+    return P8X_OK;
 }
 
 // k_mm_finish keeps a row of the output (up to 128 KB) in dynamic LDS. The attribute that allows it is per device:
@@ -712,6 +657,7 @@ static int finish_lds_attribute() {
 static int launch_mul_mat_ws(const p8x_tensor *t, const void *x, int x_dtype, int N, size_t ldx, float *y, size_t ldy, _Float16 *xr,
                              float *wmm, hipStream_t st) {
     const MmPlan p = mm_plan(t, N);
+    if (p.rg) return launch_mm_rg(t, p.rg, x, x_dtype, N, ldx, y, ldy, xr, st);
     const bool direct = p.nsplit == 1 && t->prm_identity;
     int rc;
     const dim3 agrid((t->nb + kMmActWaves - 1) / kMmActWaves, N);

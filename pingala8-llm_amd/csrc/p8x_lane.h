@@ -302,6 +302,55 @@ struct QuadSlice {
     }
 };
 
+// Payload words per lane-slice of a tile's class at run time (nw_of), for a class read from a tile word.
+__device__ __forceinline__ uint32_t nw_run(uint32_t c) { return (uint32_t)(0x18100C0A08060400ull >> (8u * c)) & 0xFFu; }
+
+// Lane offset past every buffer resource: a load there reads zeros without memory traffic.
+constexpr uint32_t kBufOob = 0x7FFFFF00u;
+
+// A lane-slice of any class of up to 4 NQ words, loaded without branches on its class: the 16-byte groups and the
+// trailing word pair that the class does not have go past the resource's records (zeros, no traffic), so a tile's
+// loads can be issued before its class decides what is done with them and every path has the same loads in flight.
+template <int NQ>
+struct AnyQuads {
+    uint32_t w[4 * NQ];
+    uint32_t p[2];
+    uint32_t s;   // fp16 row scale, zero-extended by its load
+
+    // nw = payload words of the tile's class (0: nothing is read but the scale); vs = 2 j
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rd, uint32_t toff, uint32_t nw, int hs, int j, __amdgpu_buffer_rsrc_t rs,
+                                         uint32_t soff, uint32_t vs) {
+        const uint32_t base = (uint32_t)hs * nw * 128u;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(rd, (uint32_t)q < (nw >> 2) ? base + 16u * (uint32_t)j + 512u * q : kBufOob, toff, kBufNT);
+            w[4 * q] = v[0];
+            w[4 * q + 1] = v[1];
+            w[4 * q + 2] = v[2];
+            w[4 * q + 3] = v[3];
+        }
+        const auto v = __builtin_amdgcn_raw_buffer_load_b64(rd, (nw & 2u) ? base + 512u * (nw >> 2) + 8u * (uint32_t)j : kBufOob, toff, kBufNT);
+        p[0] = v[0];
+        p[1] = v[1];
+        s = __builtin_amdgcn_raw_buffer_load_b16(rs, vs, soff, kBufNT);
+    }
+
+    // the slice as class C's (the class the words were loaded for)
+    template <int C>
+    __device__ __forceinline__ QuadSlice<C> as() const {
+        static_assert(QuadSlice<C>::NQ <= NQ, "class larger than the buffer");
+        QuadSlice<C> r;
+#pragma unroll
+        for (int i = 0; i < 4 * QuadSlice<C>::NQ; ++i) r.w[i] = w[i];
+        if constexpr (QuadSlice<C>::NP) {
+            r.w[4 * QuadSlice<C>::NQ] = p[0];
+            r.w[4 * QuadSlice<C>::NQ + 1] = p[1];
+        }
+        r.s = s;
+        return r;
+    }
+};
+
 // ------------------------------------------------------------------------------------------------ any class
 // Raw payload words of one lane-slice (any class up to NWMAX words), plus the lane's fp16 row scale: issued ahead
 // of use, then decoded into an AnySlice (labels, trellis).
