@@ -50,20 +50,6 @@ __global__ __launch_bounds__(64 * kMmActWaves) void k_mm_act(const XT *__restric
 }
 
 // ------------------------------------------------------------------------------------------------ pass 2
-struct MmJob {
-    const uint32_t *M; const uint16_t *S; const uint32_t *D;
-    const _Float16 *xr;     // x' [N][K]
-    float *y; unsigned ldy; // direct output (original rows = sorted rows, one K range)
-    float *ws;              // sorted-row planes [nsplit][N][rows] otherwise
-    const uint32_t *a2;     // [2][256] coset table words (A[f] + h c), h-major, then the same as fp16: entry 2 f + h,
-                            // 4 halves
-    int N, rows, K, nb, ng;
-    int tiles_m, tiles_n, nsplit, kper, direct;
-#ifdef P8X_TIMELINE
-    unsigned long long *tl;
-#endif
-};
-
 // Tile shape (one wave per SIMD, four per workgroup): a wave holds NTI x NTJ MFMA tiles of 32 tokens x 32 weight
 // rows, 16 NTI NTJ fp32 accumulators per lane, for all the workgroup's tokens and its own 32 NTJ rows. Each decoded
 // B operand feeds NTI MFMAs, so the decode work per MFMA falls as 1 / NTI: the class-3 kernel takes 8 x 2 (256
@@ -71,10 +57,6 @@ struct MmJob {
 // more registers, 4 x 2.
 // The class-3 kernel comes in two tile shapes, 8 x 2 and 4 x 2 (256 x 256 and 128 x 256 workgroup tiles); the plan
 // picks the one with the lower modelled time (the smaller tile halves the K-split planes a shape may need).
-__host__ __device__ constexpr int mm_waves() { return 4; }
-__host__ __device__ constexpr int mm_ntj() { return 2; }
-__host__ __device__ constexpr int mm_rows() { return 32 * mm_ntj() * mm_waves(); }
-__host__ __device__ constexpr int mm_tok(int nti) { return 32 * nti; }
 // Coset table copies in LDS: the every-class kernel's decode reads 32, one per lane of a half-wave (conflict-free);
 // the class-3 kernels keep 16 (lane j reads copy j & 15: word f 32 + h 16 + (j & 15), the 32-copy byte address with
 // the lane field doubled, halved), half the table to build per workgroup, and room next to the 8 x 2 shape's two
@@ -89,43 +71,6 @@ __host__ __device__ constexpr int mm_tab_shift(int cm) { return cm == kMmCmC3 ? 
 __host__ __device__ constexpr bool mm_f16_tab(int cm, int nti) { return cm == kMmCmC3 && nti == 4; }
 __host__ __device__ constexpr int mm_tab_words(int cm, int nti) { return mm_f16_tab(cm, nti) ? kTabWords : mm_tab_words(cm); }
 
-
-// x' half-block tile in LDS: half sh of block b holds, per token, columns 128 kh + 64 sh + 8 c8 + (0..7) as
-// chunk c = 8 kh + c8 at position c ^ (t & 15) of the token's 256-byte row, so the 16-byte operand reads of
-// 16 consecutive tokens cover all 64 banks once. TOK tokens: TOK x 128 halves per buffer.
-
-// Stage half sh of block b in two parts: mm_fetch loads it into registers, mm_put writes it to LDS. With IPW =
-// TOK / (4 NWAVES) rows of four tokens per wave, row i of wave w holds token rows 4 (IPW w + i) + (0..3); lane l
-// carries token row + (l >> 4), position l & 15 and writes it at the row's LDS base + 16 l bytes. (Direct-to-LDS loads
-// would save the registers, but while one may be in flight the compiler waits for every LDS read to finish
-// before using any, which serializes the operand reads of consecutive MFMA steps.)
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-template <int NWAVES, int TOK>
-struct XStage {
-    static constexpr int IPW = TOK / (4 * NWAVES);
-    u32x4 v[IPW];   // a native vector type: kept in registers (HIP's uint4 struct made the array a stack object)
-};
-
-template <int NWAVES, int TOK>
-__device__ __forceinline__ void mm_fetch(const MmJob &J, XStage<NWAVES, TOK> &xs, int tok0, int b, int sh, int w, int lane) {
-    constexpr int IPW = XStage<NWAVES, TOK>::IPW;
-#pragma unroll
-    for (int i = 0; i < IPW; ++i) {
-        const int row = 4 * (IPW * w + i), t = row + (lane >> 4);
-        const int ts = min(tok0 + t, J.N - 1);   // rows past N repeat the last token (never written out)
-        const int c = (lane & 15) ^ (t & 15);
-        xs.v[i] = *reinterpret_cast<const u32x4 *>(J.xr + (size_t)ts * J.K + 256 * b + 128 * (c >> 3) + 64 * sh + 8 * (c & 7));
-    }
-    __asm__ volatile("" ::: "memory");   // issued here, ahead of the products they overlap
-}
-
-// rows I0 .. I1 - 1 of the wave's share
-template <int NWAVES, int TOK, int I0 = 0, int I1 = XStage<NWAVES, TOK>::IPW>
-__device__ __forceinline__ void mm_put(const XStage<NWAVES, TOK> &xs, _Float16 *xb, int w, int lane) {
-    constexpr int IPW = XStage<NWAVES, TOK>::IPW;
-#pragma unroll
-    for (int i = I0; i < I1; ++i) *reinterpret_cast<u32x4 *>(xb + 4 * (IPW * w + i) * 128 + 8 * lane) = xs.v[i];
-}
 
 // issue the raw payload loads of the wave's NTJ tiles at block b
 template <int CM, int NWMAX, int NTJ>
@@ -569,6 +514,7 @@ static int grow(void **p, size_t *have, size_t need, const char *what) {
 
 struct MmPlan {
     int rg;    // 32-token tiles of the row-group GEMM (p8x_mm_rg.hip), which writes y itself; 0: k_mm, below
+    bool dense;   // decode the weights once (k_mm_decode), then k_mm_dense; else k_mm
     int nti;   // token tiles per wave: the workgroup tile is 256 rows x 32 nti tokens
     int tiles_m, tiles_n, nsplit, kper;
 };
@@ -589,47 +535,57 @@ static MmPlan mm_plan(const p8x_tensor *t, int N) {
     // plan (and returns the same bits) as p8x_mul_mat wherever it runs at all
     const size_t xb = ((size_t)N * t->K * sizeof(_Float16) + 255) & ~(size_t)255;
     const size_t cap = xb < (size_t)P8X_NOALLOC_SCRATCH_BYTES ? (size_t)P8X_NOALLOC_SCRATCH_BYTES - xb : 0;
-    MmPlan best{mm_rg_tiles(t, N), 4, 0, 0, 1, t->nb};
+    MmPlan best{mm_rg_tiles(t, N), false, 4, 0, 0, 1, t->nb};
     if (best.rg) return best;
     double best_cost = -1.0;
-    for (int nti = 8; nti >= 4; nti -= 4) {
-        if (nti == 8 && !c3) continue;   // the every-class decode needs the registers of the 4 x 2 shape
-        // one K block of one workgroup tile and the prologue, us (class 3: 256 x 256 and 256 x 128 measured; every
-        // class: 256 x 128)
-        const double block_us = nti == 8 ? 7.5 : c3 ? 3.9 : 4.4, pro_us = c3 ? 3.7 : 5.0;
+    auto consider = [&](bool dense, int nti, double block_us, double pro_us, double extra_us) {
         const int tiles_m = (t->rows + mm_rows() - 1) / mm_rows(), tiles_n = (N + mm_tok(nti) - 1) / mm_tok(nti);
         const long base = (long)tiles_m * tiles_n;
         for (int ns = 1; ns <= std::min(t->nb, 16); ++ns) {
             const int kper = (t->nb + ns - 1) / ns, nsr = (t->nb + kper - 1) / kper;
             if (nsr > 1 && (size_t)nsr * N * t->rows * 4 > cap) continue;
             const bool planes = nsr > 1 || !t->prm_identity;
-            const double cost = (double)((base * nsr + slots - 1) / slots) * (pro_us + kper * block_us) + (planes ? nsr * plane_us + finish_us : 0.0);
-            if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = MmPlan{0, nti, tiles_m, tiles_n, nsr, kper}; }
+            const double cost = (double)((base * nsr + slots - 1) / slots) * (pro_us + kper * block_us) + (planes ? nsr * plane_us + finish_us : 0.0) + extra_us;
+            if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = MmPlan{0, dense, nti, tiles_m, tiles_n, nsr, kper}; }
         }
-    }
+    };
+    // One K block of one workgroup tile and the prologue, us, measured: class 3 at 256 x 256 and 256 x 128; every class
+    // at 256 x 128 (its decode needs the registers; 7.4 with the released ffn_down mix of classes 2, 3 and 4).
+    if (c3) consider(false, 8, 7.5, 3.7, 0.0);
+    consider(false, 4, c3 ? 3.9 : 7.4, c3 ? 3.7 : 5.0, 0.0);
+    // Decoded operands: a launch that writes 16 KB per tile (33 us for 117 MB), then 0.9 us per 32 tokens and block with
+    // every CU busy. 4096 x 14336, the ffn_down mix, 1500 tokens: k_mm 427 us a call, 276 here (two K ranges, 192-token
+    // tiles; the dense kernel alone 1.07 PFLOP/s, the card's library product 1.2). Class 3, 14336 x 4096: 512 tokens 98
+    // (k_mm) and 123 us, 2048 tokens 394 and 399, so class 3 keeps k_mm nearly everywhere. Class-0 tiles are skipped by
+    // k_mm and have no operands: tensors with such tiles keep it.
+    if (!t->class_tiles[0])
+        for (int nti = 4; nti <= 6; ++nti) consider(true, nti, nti == 4 ? 3.6 : nti == 5 ? 4.7 : 5.8, 2.0, 5.0 + mm_dense_w_bytes(t) / 4.2e6);
     return best;
 }
 
 // workspace bytes of one prompt GEMM call: rotated fp16 activations ([N][K], or whole 32-token tiles), and (k_mm with a
 // K split or rows to un-permute) the sorted-row output planes [nsplit][N][rows] f32
-static void mm_workspace(const p8x_tensor *t, int N, size_t *x_bytes, size_t *plane_bytes) {
+static void mm_workspace(const p8x_tensor *t, int N, size_t *x_bytes, size_t *plane_bytes, size_t *w_bytes) {
     const MmPlan p = mm_plan(t, N);
     *x_bytes = p.rg ? mm_rg_x_bytes(t, p.rg) : (size_t)N * t->K * sizeof(_Float16);
     *plane_bytes = p.rg || (p.nsplit == 1 && t->prm_identity) ? 0 : (size_t)p.nsplit * N * t->rows * 4;
+    *w_bytes = p.dense ? mm_dense_w_bytes(t) : 0;
 }
 
 int reserve_mul_mat(const p8x_tensor *t, int n_max) {
     p8x_tensor *tw = const_cast<p8x_tensor *>(t);
-    size_t xb = 0, planes = 0;   // the largest needs over every N <= n_max (the split count depends on N)
+    size_t xb = 0, planes = 0, wb = 0;   // the largest needs over every N <= n_max (the split count depends on N)
     for (int n = 1; n <= n_max; ++n) {
-        size_t x1, p1;
-        mm_workspace(t, n, &x1, &p1);
+        size_t x1, p1, w1;
+        mm_workspace(t, n, &x1, &p1, &w1);
         xb = std::max(xb, x1);
         planes = std::max(planes, p1);
+        wb = std::max(wb, w1);
     }
     int rc;
     if ((rc = grow((void **)&tw->wx16, &tw->wx16_elems, xb, "p8x_mul_mat_reserve: activation workspace"))) return rc;
     if (planes && (rc = grow((void **)&tw->wmm, &tw->wmm_bytes, planes, "p8x_mul_mat_reserve: output planes"))) return rc;
+    if (wb && (rc = grow(&tw->wbw, &tw->wbw_bytes, wb, "p8x_mul_mat_reserve: decoded weights"))) return rc;
     return P8X_OK;
 }
 
@@ -652,14 +608,19 @@ static int finish_lds_attribute() {
 }
 
 // the launches of one prompt GEMM with its workspace given: xr >= N K fp16, wmm >= the plane bytes (unused when the
-// output is written directly)
-
+// output is written directly), bw the decoded operands' bytes. Without bw a decoded-weights plan runs k_mm with that
+// plan's K split: the same bits.
 static int launch_mul_mat_ws(const p8x_tensor *t, const void *x, int x_dtype, int N, size_t ldx, float *y, size_t ldy, _Float16 *xr,
-                             float *wmm, hipStream_t st) {
-    const MmPlan p = mm_plan(t, N);
+                             float *wmm, void *bw, hipStream_t st) {
+    MmPlan p = mm_plan(t, N);
     if (p.rg) return launch_mm_rg(t, p.rg, x, x_dtype, N, ldx, y, ldy, xr, st);
     const bool direct = p.nsplit == 1 && t->prm_identity;
     int rc;
+    if (p.dense && !bw) {
+        p.dense = false;
+        p.nti = 4;
+        p.tiles_n = (N + mm_tok(p.nti) - 1) / mm_tok(p.nti);
+    }
     const dim3 agrid((t->nb + kMmActWaves - 1) / kMmActWaves, N);
     if (x_dtype == P8X_F32) hipLaunchKernelGGL(k_mm_act<float>, agrid, dim3(64 * kMmActWaves), 0, st, (const float *)x, ldx, t->ic, t->K, xr);
     else hipLaunchKernelGGL(k_mm_act<uint16_t>, agrid, dim3(64 * kMmActWaves), 0, st, (const uint16_t *)x, ldx, t->ic, t->K, xr);
@@ -672,8 +633,11 @@ static int launch_mul_mat_ws(const p8x_tensor *t, const void *x, int x_dtype, in
 #ifdef P8X_TIMELINE
     J.tl = timeline_buf();
 #endif
+    J.bw = (const _Float16 *)bw;
     const int grid = ((p.tiles_m * p.tiles_n * p.nsplit + kXcds - 1) / kXcds) * kXcds;
-    if (!mm_only_c3(t)) hipLaunchKernelGGL((k_mm<kMmCmAll, 4>), dim3(grid), dim3(64 * mm_waves()), 0, st, J);
+    if (p.dense) {
+        if ((rc = launch_mm_decode(t, bw, st)) || (rc = launch_mm_dense(p.nti, J, st))) return rc;
+    } else if (!mm_only_c3(t)) hipLaunchKernelGGL((k_mm<kMmCmAll, 4>), dim3(grid), dim3(64 * mm_waves()), 0, st, J);
     else if (p.nti == 8) hipLaunchKernelGGL((k_mm<kMmCmC3, 8>), dim3(grid), dim3(64 * mm_waves()), 0, st, J);
     else hipLaunchKernelGGL((k_mm<kMmCmC3, 4>), dim3(grid), dim3(64 * mm_waves()), 0, st, J);
     if ((rc = hip_check(hipGetLastError(), "k_mm launch"))) return rc;
@@ -701,12 +665,13 @@ static int launch_mul_mat_ws(const p8x_tensor *t, const void *x, int x_dtype, in
 int launch_mul_mat(const p8x_tensor *t, const void *x, int x_dtype, int N, size_t ldx, float *y, size_t ldy, hipStream_t st) {
     if (((uintptr_t)x & 15) || (ldx % 8)) return set_error(P8X_ERR_ARG, "p8x_mul_mat: x must be 16-byte aligned with ldx %% 8 == 0");
     p8x_tensor *tw = const_cast<p8x_tensor *>(t);
-    size_t xb, pb;
-    mm_workspace(t, N, &xb, &pb);
+    size_t xb, pb, wb;
+    mm_workspace(t, N, &xb, &pb, &wb);
     int rc;
+    if (wb && (rc = grow(&tw->wbw, &tw->wbw_bytes, wb, "p8x_mul_mat: decoded weights"))) return rc;
     if ((rc = grow((void **)&tw->wx16, &tw->wx16_elems, xb, "p8x_mul_mat: activation workspace"))) return rc;
     if (pb && (rc = grow((void **)&tw->wmm, &tw->wmm_bytes, pb, "p8x_mul_mat: output planes"))) return rc;
-    return launch_mul_mat_ws(t, x, x_dtype, N, ldx, y, ldy, reinterpret_cast<_Float16 *>(tw->wx16), tw->wmm, st);
+    return launch_mul_mat_ws(t, x, x_dtype, N, ldx, y, ldy, reinterpret_cast<_Float16 *>(tw->wx16), tw->wmm, wb ? tw->wbw : nullptr, st);
 }
 
 // ------------------------------------------------------------------------------------------------ no-allocation variant
@@ -747,8 +712,8 @@ extern "C" int p8x_mul_mat_noalloc(const p8x_tensor *t, const void *x, int x_dty
     if (x_dtype != P8X_F32 && x_dtype != P8X_BF16) return set_error(P8X_ERR_ARG, "p8x_mul_mat_noalloc: x dtype %d", x_dtype);
     if (N < 1 || ldx < (size_t)t->K || ldy < (size_t)t->rows) return set_error(P8X_ERR_ARG, "p8x_mul_mat_noalloc: N %d ldx %zu ldy %zu", N, ldx, ldy);
     if (((uintptr_t)x & 15) || (ldx % 8)) return set_error(P8X_ERR_ARG, "p8x_mul_mat_noalloc: x must be 16-byte aligned with ldx %% 8 == 0");
-    size_t xb, pb;
-    mm_workspace(t, N, &xb, &pb);
+    size_t xb, pb, wb;
+    mm_workspace(t, N, &xb, &pb, &wb);
     const size_t xb_al = (xb + 255) & ~(size_t)255;
     if (xb_al + pb > (size_t)P8X_NOALLOC_SCRATCH_BYTES)
         return set_error(P8X_ERR_UNSUPPORTED, "p8x_mul_mat_noalloc: %d tokens of a %d x %d tensor need %zu workspace bytes, above the %d-byte scratch",
@@ -759,7 +724,10 @@ extern "C" int p8x_mul_mat_noalloc(const p8x_tensor *t, const void *x, int x_dty
         if (rc) return rc;
         base = static_cast<uint8_t *>(scratch_ptr(t->device));
     }
-    // x' first, the output planes after it on a 256-byte boundary; every byte read is written earlier in the call
-    return launch_mul_mat_ws(t, x, x_dtype, N, ldx, y, ldy, reinterpret_cast<_Float16 *>(base), reinterpret_cast<float *>(base + xb_al),
+    // x' first, the output planes after it on a 256-byte boundary, then the decoded weights where they fit (k_mm
+    // otherwise, the same bits); every byte read is written earlier in the call
+    const size_t w_off = (xb_al + pb + 255) & ~(size_t)255;
+    void *bw = wb && w_off + wb <= (size_t)P8X_NOALLOC_SCRATCH_BYTES ? base + w_off : nullptr;
+    return launch_mul_mat_ws(t, x, x_dtype, N, ldx, y, ldy, reinterpret_cast<_Float16 *>(base), reinterpret_cast<float *>(base + xb_al), bw,
                              (hipStream_t)stream);
 }

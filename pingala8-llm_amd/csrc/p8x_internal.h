@@ -60,6 +60,8 @@ struct p8x_tensor {
     size_t wx16_elems = 0;           // capacity in bytes
     float *wmm = nullptr;            // prompt GEMM: K-split partial planes (grown on demand)
     size_t wmm_bytes = 0;
+    void *wbw = nullptr;             // prompt GEMM of many tokens: decoded fp16 operands, 2 rows K bytes (grown on demand)
+    size_t wbw_bytes = 0;
     uint32_t a2_host[512];           // host copy of a2 (batches check that tensors share the tables)
 };
 

@@ -69,11 +69,75 @@ constexpr int kMmCmC3 = 1 << 3, kMmCmAll = 0xFE;
 constexpr int kMmMain = 3;   // the class with a branch-free path in every instantiation (the 2-bit bulk)
 __host__ __device__ constexpr int mm_nwmax(int cm) { return cm == kMmCmC3 ? 8 : 24; }
 
+// ------------------------------------------------------------------------------------------------ tiled kernels
+struct MmJob {
+    const uint32_t *M; const uint16_t *S; const uint32_t *D;
+    const _Float16 *xr;     // x' [N][K]
+    float *y; unsigned ldy; // direct output (original rows = sorted rows, one K range)
+    float *ws;              // sorted-row planes [nsplit][N][rows] otherwise
+    const uint32_t *a2;     // [2][256] coset table words (A[f] + h c), h-major, then the same as fp16: entry 2 f + h,
+                            // 4 halves
+    int N, rows, K, nb, ng;
+    const _Float16 *bw;     // k_mm_dense: the decoded weights (k_mm_decode)
+    int tiles_m, tiles_n, nsplit, kper, direct;
+#ifdef P8X_TIMELINE
+    unsigned long long *tl;
+#endif
+};
+
+// workgroup tile of k_mm and k_mm_dense: four waves, one per SIMD, each 64 weight rows x all of the tile's tokens
+__host__ __device__ constexpr int mm_waves() { return 4; }
+__host__ __device__ constexpr int mm_ntj() { return 2; }
+__host__ __device__ constexpr int mm_rows() { return 32 * mm_ntj() * mm_waves(); }
+__host__ __device__ constexpr int mm_tok(int nti) { return 32 * nti; }
+
+// x' half-block tile in LDS: half sh of block b holds, per token, columns 128 kh + 64 sh + 8 c8 + (0..7) as
+// chunk c = 8 kh + c8 at position c ^ (t & 15) of the token's 256-byte row, so the 16-byte operand reads of
+// 16 consecutive tokens cover all 64 banks once. TOK tokens: TOK x 128 halves per buffer.
+
+// Stage half sh of block b in two parts: mm_fetch loads it into registers, mm_put writes it to LDS. With IPW =
+// TOK / (4 NWAVES) rows of four tokens per wave, row i of wave w holds token rows 4 (IPW w + i) + (0..3); lane l
+// carries token row + (l >> 4), position l & 15 and writes it at the row's LDS base + 16 l bytes. (Direct-to-LDS loads
+// would save the registers, but while one may be in flight the compiler waits for every LDS read to finish
+// before using any, which serializes the operand reads of consecutive MFMA steps.)
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+template <int NWAVES, int TOK>
+struct XStage {
+    static constexpr int IPW = TOK / (4 * NWAVES);
+    u32x4 v[IPW];   // a native vector type: kept in registers (HIP's uint4 struct made the array a stack object)
+};
+
+template <int NWAVES, int TOK>
+__device__ __forceinline__ void mm_fetch(const MmJob &J, XStage<NWAVES, TOK> &xs, int tok0, int b, int sh, int w, int lane) {
+    constexpr int IPW = XStage<NWAVES, TOK>::IPW;
+#pragma unroll
+    for (int i = 0; i < IPW; ++i) {
+        const int row = 4 * (IPW * w + i), t = row + (lane >> 4);
+        const int ts = min(tok0 + t, J.N - 1);   // rows past N repeat the last token (never written out)
+        const int c = (lane & 15) ^ (t & 15);
+        xs.v[i] = *reinterpret_cast<const u32x4 *>(J.xr + (size_t)ts * J.K + 256 * b + 128 * (c >> 3) + 64 * sh + 8 * (c & 7));
+    }
+    __asm__ volatile("" ::: "memory");   // issued here, ahead of the products they overlap
+}
+
+// rows I0 .. I1 - 1 of the wave's share
+template <int NWAVES, int TOK, int I0 = 0, int I1 = XStage<NWAVES, TOK>::IPW>
+__device__ __forceinline__ void mm_put(const XStage<NWAVES, TOK> &xs, _Float16 *xb, int w, int lane) {
+    constexpr int IPW = XStage<NWAVES, TOK>::IPW;
+#pragma unroll
+    for (int i = I0; i < I1; ++i) *reinterpret_cast<u32x4 *>(xb + 4 * (IPW * w + i) * 128 + 8 * lane) = xs.v[i];
+}
+
 // the row-group GEMM (p8x_mm_rg.hip): up to kMmRgMaxTokens tokens in one pass over the weights
 constexpr int kMmRgMaxTokens = 64;
 bool mm_only_c3(const p8x_tensor *t);
 int mm_rg_tiles(const p8x_tensor *t, int N);                  // 32-token tiles of the call, 0: not served
 size_t mm_rg_x_bytes(const p8x_tensor *t, int tiles);         // its x' workspace
+// the decoded-weights GEMM (p8x_mm_dense.hip): weight operands decoded once per call, then a dense kernel of
+// 256 rows x 32 nti tokens per workgroup, nti 4 .. 6
+size_t mm_dense_w_bytes(const p8x_tensor *t);
+int launch_mm_decode(const p8x_tensor *t, void *bw, hipStream_t st);
+int launch_mm_dense(int nti, const MmJob &J, hipStream_t st);
 int launch_mm_rg(const p8x_tensor *t, int tiles, const void *x, int x_dtype, int N, size_t ldx, float *y, size_t ldy, void *xf, hipStream_t st);
 
 }  // namespace p8x
