@@ -459,12 +459,32 @@ template <typename XT>
 __global__ __launch_bounds__(1024) void k_mm_finish(const float *__restrict__ ws, int nsplit, int N, int rows, const int16_t *__restrict__ pinv,
                                                     const int *__restrict__ cp, const uint16_t *__restrict__ cc, const float *__restrict__ cv,
                                                     const XT *__restrict__ x, size_t ldx, float *__restrict__ y, size_t ldy) {
-    extern __shared__ float srow[];   // [rows]
+    extern __shared__ __attribute__((aligned(16))) float srow[];   // [rows]
     const int n = blockIdx.x;
-    for (int r = threadIdx.x; r < rows; r += 1024) {
-        float v = 0.f;
-        for (int k = 0; k < nsplit; ++k) v += ws[((size_t)k * N + n) * rows + r];
-        srow[r] = v;
+    // Four rows per thread and step (rows is a multiple of 32, the planes 16-byte aligned), two or four loads in flight:
+    // a call of few tokens has few workgroups, and one load after another was most of its time (9728 rows x 19 tokens:
+    // 17 us; 4096 rows, 4 planes, 65 tokens: the whole call 40.3 -> 26.6 us).
+    auto plane = [&](int k, int r) { return as_global(reinterpret_cast<const f32x4 *>(ws + ((size_t)k * N + n) * rows))[r >> 2]; };
+    if (nsplit == 1) {
+        for (int r = 4 * threadIdx.x; r < rows; r += 8192) {
+            const bool two = r + 4096 < rows;
+            const f32x4 a = plane(0, r), b = plane(0, two ? r + 4096 : r);
+            *reinterpret_cast<f32x4 *>(srow + r) = a;
+            if (two) *reinterpret_cast<f32x4 *>(srow + r + 4096) = b;
+        }
+    } else {
+        for (int r = 4 * threadIdx.x; r < rows; r += 4096) {
+            f32x4 v = {0.f, 0.f, 0.f, 0.f};
+            for (int k0 = 0; k0 < nsplit; k0 += 4) {
+                f32x4 pv[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) pv[k] = plane(min(k0 + k, nsplit - 1), r);
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (k0 + k < nsplit) v += pv[k];
+            }
+            *reinterpret_cast<f32x4 *>(srow + r) = v;
+        }
     }
     __syncthreads();
     const XT *xr = x + (size_t)n * ldx;
@@ -555,10 +575,12 @@ static MmPlan mm_plan(const p8x_tensor *t, int N) {
     consider(false, 4, c3 ? 3.9 : 7.4, c3 ? 3.7 : 5.0, 0.0);
     // Decoded operands: a launch that writes 16 KB per tile (33 us for 117 MB), then 0.9 us per 32 tokens and block with
     // every CU busy. 4096 x 14336, the ffn_down mix, 1500 tokens: k_mm 427 us a call, 276 here (two K ranges, 192-token
-    // tiles; the dense kernel alone 1.07 PFLOP/s, the card's library product 1.2). Class 3, 14336 x 4096: 512 tokens 98
-    // (k_mm) and 123 us, 2048 tokens 394 and 399, so class 3 keeps k_mm nearly everywhere. Class-0 tiles are skipped by
-    // k_mm and have no operands: tensors with such tiles keep it.
-    if (!t->class_tiles[0])
+    // Decoded operands: a launch that writes 16 KB per tile (33 us for 117 MB), then 0.9 us per 32 tokens and block with
+    // every CU busy. 4096 x 14336, the ffn_down mix, 1500 tokens: k_mm 443 us a call, 237 here (two K ranges, 192-token
+    // tiles; the dense kernel alone 1.07 PFLOP/s, the card's library product 1.2). Class 3 keeps k_mm, whose decode is
+    // cheaper: 14336 x 4096, 512 tokens 98 (k_mm) and 123 us, 2048 tokens 394 and 399. Class-0 tiles are skipped by k_mm
+    // and have no operands: tensors with such tiles keep it.
+    if (!c3 && !t->class_tiles[0])
         for (int nti = 4; nti <= 6; ++nti) consider(true, nti, nti == 4 ? 3.6 : nti == 5 ? 4.7 : 5.8, 2.0, 5.0 + mm_dense_w_bytes(t) / 4.2e6);
     return best;
 }

@@ -28,7 +28,7 @@ struct MmDecJob {
     uint32_t dbytes, sbytes;
 };
 
-template <int CM, int C>
+template <int C>
 __device__ __forceinline__ void mm_decode_tile(const uint32_t *tab, const QuadSlice<C> &p, uint32_t bankbytes, gptr<half8v> out) {
     const uint32_t H = p.coset_bits();
     const half2v s2 = {__builtin_bit_cast(_Float16, (uint16_t)p.s), __builtin_bit_cast(_Float16, (uint16_t)p.s)};
@@ -39,16 +39,10 @@ __device__ __forceinline__ void mm_decode_tile(const uint32_t *tab, const QuadSl
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             const uint32_t a = p.template addr<0>(2 * s + u, hq);
-            if constexpr (CM == kMmCmC3) {
-                const uint2 e = *reinterpret_cast<const uint2 *>(reinterpret_cast<const char *>(tab) + a);
-                v[2 * u] = __builtin_bit_cast(half2v, e.x) * s2;
-                v[2 * u + 1] = __builtin_bit_cast(half2v, e.y) * s2;
-            } else {
-                uint32_t w[3] = {lds_word(tab, a), 0u, 0u};
-                if constexpr (nstage_of(C) > 1) w[1] = lds_word(tab, p.template addr<1>(2 * s + u, hq));
-                if constexpr (nstage_of(C) > 2) w[2] = lds_word(tab, p.template addr<2>(2 * s + u, hq));
-                weights_chunk<C>(w, s2, v[2 * u], v[2 * u + 1]);
-            }
+            uint32_t w[3] = {lds_word(tab, a), 0u, 0u};
+            if constexpr (nstage_of(C) > 1) w[1] = lds_word(tab, p.template addr<1>(2 * s + u, hq));
+            if constexpr (nstage_of(C) > 2) w[2] = lds_word(tab, p.template addr<2>(2 * s + u, hq));
+            weights_chunk<C>(w, s2, v[2 * u], v[2 * u + 1]);
         }
         half8v B;
 #pragma unroll
@@ -59,13 +53,12 @@ __device__ __forceinline__ void mm_decode_tile(const uint32_t *tab, const QuadSl
 
 // One tile per wave and step, the next tile's payload in flight. Two workgroups per CU (64 KB table each); bound by
 // its stores (16 KB per 2.1 KB tile read), which are non-temporal: 28 to 34 us for 117 MB (36 to 38 as plain stores).
-template <int CM>
 __global__ __launch_bounds__(64 * kMmDecWaves) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_mm_decode(MmDecJob J) {
-    constexpr int NT = 64 * kMmDecWaves, NQ = CM == kMmCmC3 ? 2 : 6;
+    constexpr int NT = 64 * kMmDecWaves, NQ = 6;
     __shared__ uint32_t tab[kTabWords];   // LDS address 0
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 31, kh = lane >> 5;
-    const uint32_t bankbytes = (uint32_t)((CM == kMmCmC3 ? (j & 15) << 1 : j) << 2) * 0x01010101u;
+    const uint32_t bankbytes = (uint32_t)(j << 2) * 0x01010101u;
     const int nw = (int)gridDim.x * kMmDecWaves;
     int t = (int)blockIdx.x * kMmDecWaves + w;
     const __amdgpu_buffer_rsrc_t rd = buffer_rsrc(J.D, J.dbytes), rs = buffer_rsrc(J.Sg, J.sbytes);
@@ -80,42 +73,30 @@ __global__ __launch_bounds__(64 * kMmDecWaves) __attribute__((amdgpu_waves_per_e
     issue(t);
     constexpr int TPT = kTabWords / 4 / NT;
     uint4 *t4 = reinterpret_cast<uint4 *>(tab);
-    if constexpr (CM == kMmCmC3) {   // 16 copies of the fp16 entries
-        const uint2 *e16 = reinterpret_cast<const uint2 *>(J.a2 + 512);
-        uint2 v[TPT];
+    // 32 copies of the table words, bytes offset by 128
+    uint32_t v[TPT];
 #pragma unroll
-        for (int k = 0; k < TPT; ++k) v[k] = e16[(tid + k * NT) >> 3];
-#pragma unroll
-        for (int k = 0; k < TPT; ++k) t4[tid + k * NT] = make_uint4(v[k].x, v[k].y, v[k].x, v[k].y);
-    } else {                         // 32 copies of the words, bytes offset by 128
-        uint32_t v[TPT];
-#pragma unroll
-        for (int k = 0; k < TPT; ++k) {
-            const int i = tid + k * NT;
-            v[k] = J.a2[((i >> 3) & 1) * 256 + (i >> 4)] ^ 0x80808080u;
-        }
-#pragma unroll
-        for (int k = 0; k < TPT; ++k) t4[tid + k * NT] = make_uint4(v[k], v[k], v[k], v[k]);
+    for (int k = 0; k < TPT; ++k) {
+        const int i = tid + k * NT;
+        v[k] = J.a2[((i >> 3) & 1) * 256 + (i >> 4)] ^ 0x80808080u;
     }
+#pragma unroll
+    for (int k = 0; k < TPT; ++k) t4[tid + k * NT] = make_uint4(v[k], v[k], v[k], v[k]);
     __syncthreads();
     for (; t < J.nt; t += nw) {
         const AnyQuads<NQ> cur = nxt;
         const uint32_t c = cn;
         issue(t + nw);
         const gptr<half8v> out = as_global_rw(reinterpret_cast<half8v *>(J.bw + (size_t)t * kMmTileHalves)) + lane;
-        if constexpr (CM == kMmCmC3) {
-            mm_decode_tile<CM>(tab, cur.template as<3>(), bankbytes, out);
-        } else {
-            switch (c) {
-                case 1: mm_decode_tile<CM>(tab, cur.template as<1>(), bankbytes, out); break;
-                case 2: mm_decode_tile<CM>(tab, cur.template as<2>(), bankbytes, out); break;
-                case 3: mm_decode_tile<CM>(tab, cur.template as<3>(), bankbytes, out); break;
-                case 4: mm_decode_tile<CM>(tab, cur.template as<4>(), bankbytes, out); break;
-                case 5: mm_decode_tile<CM>(tab, cur.template as<5>(), bankbytes, out); break;
-                case 6: mm_decode_tile<CM>(tab, cur.template as<6>(), bankbytes, out); break;
-                case 7: mm_decode_tile<CM>(tab, cur.template as<7>(), bankbytes, out); break;
-                default: break;   // no class-0 tiles here (mm_plan)
-            }
+        switch (c) {
+            case 1: mm_decode_tile(tab, cur.template as<1>(), bankbytes, out); break;
+            case 2: mm_decode_tile(tab, cur.template as<2>(), bankbytes, out); break;
+            case 3: mm_decode_tile(tab, cur.template as<3>(), bankbytes, out); break;
+            case 4: mm_decode_tile(tab, cur.template as<4>(), bankbytes, out); break;
+            case 5: mm_decode_tile(tab, cur.template as<5>(), bankbytes, out); break;
+            case 6: mm_decode_tile(tab, cur.template as<6>(), bankbytes, out); break;
+            case 7: mm_decode_tile(tab, cur.template as<7>(), bankbytes, out); break;
+            default: break;   // no class-0 tiles here (mm_plan)
         }
     }
 }
@@ -232,8 +213,7 @@ size_t mm_dense_w_bytes(const p8x_tensor *t) { return t->nt * kMmTileHalves * si
 int launch_mm_decode(const p8x_tensor *t, void *bw, hipStream_t st) {
     MmDecJob J{t->M, t->Sg, t->D, t->a2, (_Float16 *)bw, (int)t->nt, (uint32_t)(t->kbytes - offset_D(t->nt)), (uint32_t)(t->nb * t->rows * 2)};
     const int grid = std::min((int)((t->nt + kMmDecWaves - 1) / kMmDecWaves), 2 * num_cus());
-    if (mm_only_c3(t)) hipLaunchKernelGGL((k_mm_decode<kMmCmC3>), dim3(grid), dim3(64 * kMmDecWaves), 0, st, J);
-    else hipLaunchKernelGGL((k_mm_decode<kMmCmAll>), dim3(grid), dim3(64 * kMmDecWaves), 0, st, J);
+    hipLaunchKernelGGL(k_mm_decode, dim3(grid), dim3(64 * kMmDecWaves), 0, st, J);
     return hip_check(hipGetLastError(), "k_mm_decode launch");
 }
 

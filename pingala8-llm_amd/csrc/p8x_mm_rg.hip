@@ -51,36 +51,49 @@ struct MmRgJob {
 // class 3 with one token tile: 16 waves at 128 VGPRs; two tiles or any class: 8 waves at 256
 __host__ __device__ constexpr int mm_rg_waves(int cm, int tt) { return cm == kMmCmC3 && tt == 1 ? 16 : 8; }
 
-// half h (steps 8 h .. 8 h + 7) of one tile: decode a step's operand, multiply it with every token tile's
-template <int CM, int C, int T>
-__device__ __forceinline__ void mm_rg_half(const uint32_t *tab, const QuadSlice<C> &p, uint32_t H, uint32_t bankbytes, half2v s2, int h,
-                                           const half8v (&A)[8][T], float16v (&acc)[T]) {
-#pragma unroll
-    for (int s8 = 0; s8 < 8; ++s8) {
-        const int s = 8 * h + s8;
+// A wave's x' operands are loaded a segment of steps ahead: SEG steps x T token tiles = 8 operands, 32 registers.
+__host__ __device__ constexpr int mm_rg_seg(int tt) { return 8 / tt; }
+
+// table words of step s (two chunks), and the step's operand from them
+template <int CM, int C>
+struct MmRgWords {
+    uint32_t w[2][CM == kMmCmC3 ? 2 : nstage_of(C)];
+    __device__ __forceinline__ void load(const uint32_t *tab, const QuadSlice<C> &p, uint32_t H, uint32_t bankbytes, int s) {
         const uint32_t hq = coset_bytes(H, bankbytes, s >> 1);
-        half2v v[4];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             const uint32_t a = p.template addr<0>(2 * s + u, hq);
             if constexpr (CM == kMmCmC3) {   // fp16 table entry: the chunk's four weights
                 const uint2 e = *reinterpret_cast<const uint2 *>(reinterpret_cast<const char *>(tab) + a);
-                v[2 * u] = __builtin_bit_cast(half2v, e.x) * s2;
-                v[2 * u + 1] = __builtin_bit_cast(half2v, e.y) * s2;
+                w[u][0] = e.x;
+                w[u][1] = e.y;
             } else {
-                uint32_t w[3] = {lds_word(tab, a), 0u, 0u};
-                if constexpr (nstage_of(C) > 1) w[1] = lds_word(tab, p.template addr<1>(2 * s + u, hq));
-                if constexpr (nstage_of(C) > 2) w[2] = lds_word(tab, p.template addr<2>(2 * s + u, hq));
-                weights_chunk<C>(w, s2, v[2 * u], v[2 * u + 1]);
+                w[u][0] = lds_word(tab, a);
+                if constexpr (nstage_of(C) > 1) w[u][1] = lds_word(tab, p.template addr<1>(2 * s + u, hq));
+                if constexpr (nstage_of(C) > 2) w[u][2] = lds_word(tab, p.template addr<2>(2 * s + u, hq));
+            }
+        }
+    }
+    __device__ __forceinline__ half8v operand(half2v s2) const {
+        half2v v[4];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if constexpr (CM == kMmCmC3) {
+                v[2 * u] = __builtin_bit_cast(half2v, w[u][0]) * s2;
+                v[2 * u + 1] = __builtin_bit_cast(half2v, w[u][1]) * s2;
+            } else {
+                uint32_t x[3] = {w[u][0], 0u, 0u};
+                if constexpr (nstage_of(C) > 1) x[1] = w[u][1];
+                if constexpr (nstage_of(C) > 2) x[2] = w[u][2];
+                weights_chunk<C>(x, s2, v[2 * u], v[2 * u + 1]);
             }
         }
         half8v B;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { B[2 * i] = v[i].x; B[2 * i + 1] = v[i].y; }
-#pragma unroll
-        for (int t = 0; t < T; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[s8][t], B, acc[t], 0, 0, 0);
+        for (int k = 0; k < 4; ++k) { B[2 * k] = v[k].x; B[2 * k + 1] = v[k].y; }
+        return B;
     }
-}
+};
 
 template <int CM, int T>
 __global__ __launch_bounds__(64 * mm_rg_waves(CM, T)) __attribute__((amdgpu_waves_per_eu(mm_rg_waves(CM, T) / 4, mm_rg_waves(CM, T) / 4)))
@@ -109,17 +122,19 @@ void k_mm_rg(MmRgJob J) {
             r.load(rd, toff, nw_run(c), kh, j, rs, soff, 2u * j);
         }
     };
-    auto issue_a = [&](half8v (&A)[8][T], int b, int h) {
+    constexpr int SEG = mm_rg_seg(T);
+    auto issue_a = [&](half8v (&A)[SEG][T], int b, int q) {
         const int bi = min(b, J.nb - 1);
-        const gptr<const half8v> p = as_global(reinterpret_cast<const half8v *>(J.xf)) + ((size_t)bi * 16 + 8 * h) * T * 64 + lane;
+        const gptr<const half8v> p = as_global(reinterpret_cast<const half8v *>(J.xf)) + ((size_t)bi * 16 + SEG * q) * T * 64 + lane;
 #pragma unroll
-        for (int s = 0; s < 8; ++s)
+        for (int s = 0; s < SEG; ++s)
 #pragma unroll
             for (int t = 0; t < T; ++t) A[s][t] = p[(s * T + t) * 64];
+        __asm__ volatile("" ::: "memory");   // issued here, ahead of the products they overlap
     };
     Raw nxt;
     uint32_t cn;
-    half8v A0[8][T], A1[8][T];
+    half8v A0[SEG][T], A1[SEG][T];
     int g = (int)blockIdx.x + min(team, J.gc - 1) * gstep;
     // the first tile's loads and the table's go out together
     issue_raw(nxt, cn, g, b0);
@@ -160,13 +175,30 @@ void k_mm_rg(MmRgJob J) {
                 const int gn = last ? g + gstep * J.gc : g, bn = last ? b0 : b + 1;
                 issue_a(A1, b, 1);
                 issue_raw(nxt, cn, gn, bn);
+                __asm__ volatile("" ::: "memory");
                 const half2v s2 = {__builtin_bit_cast(_Float16, (uint16_t)cur.s), __builtin_bit_cast(_Float16, (uint16_t)cur.s)};
                 auto tile = [&](auto cls, const auto &p) {
                     constexpr int C = decltype(cls)::value;
                     const uint32_t H = p.coset_bits();
-                    mm_rg_half<CM, C, T>(tab, p, H, bankbytes, s2, 0, A0, acc);
-                    issue_a(A0, bn, 0);
-                    mm_rg_half<CM, C, T>(tab, p, H, bankbytes, s2, 1, A1, acc);
+                    MmRgWords<CM, C> W[2];   // the next step's table words are read before this step's products
+                    W[0].load(tab, p, H, bankbytes, 0);
+#pragma unroll
+                    for (int st = 0; st < 16; ++st) {
+                        const int q = st / SEG, i = st % SEG;
+                        if (st < 15) W[(st + 1) & 1].load(tab, p, H, bankbytes, st + 1);
+                        const half8v B = W[st & 1].operand(s2);
+#pragma unroll
+                        for (int t = 0; t < T; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16((q & 1) ? A1[i][t] : A0[i][t], B, acc[t], 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);   // one step's table words ahead, no more: bounds the live registers
+                        if (i == SEG - 1) {   // the segment's registers take the one two ahead (the next tile's first two at the end)
+                            if (q & 1) {
+                                if (q + 2 < 2 * T) issue_a(A1, b, q + 2);
+                            } else {
+                                if (q + 2 < 2 * T) issue_a(A0, b, q + 2);
+                                else issue_a(A0, bn, 0);
+                            }
+                        }
+                    }
                 };
                 if constexpr (CM == kMmCmC3) {
                     tile(std::integral_constant<int, 3>{}, cur);
@@ -194,7 +226,14 @@ void k_mm_rg(MmRgJob J) {
         if (active)
             for (int i = wk; i < 16 * T; i += wpg) {
                 float v = 0.f;
-                for (int k = 0; k < wpg; ++k) v += red[team * wpg + k][i][lane];
+                for (int k0 = 0; k0 < wpg; k0 += 4) {   // four reads in flight, added in wave order
+                    float pv[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) pv[k] = red[team * wpg + min(k0 + k, wpg - 1)][i][lane];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (k0 + k < wpg) v += pv[k];
+                }
                 const int q = i & 15, tok = 32 * (i >> 4) + 8 * (q >> 2) + 4 * kh + (q & 3), r = ro & 0x7FFF;
                 if (tok >= J.N) continue;
                 if (ro & 0x8000)
