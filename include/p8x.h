@@ -127,14 +127,15 @@ int p8x_vec_dot(const p8x_tensor *t, int act, const void *q, const float *d, int
 int p8x_vec_dot_rows(const p8x_tensor *t, int act, const void *q, const float *d, int ncols, int g0, int ng, const float *x, size_t ldx,
                      float *y, size_t ldy, int32_t *partials, void *stream);
 /* y = W x for 1..8 columns (vr_mul_mat_vec, CPU.patch:4466-4521): activation prep + fused decode-GEMV +
- * un-permute + clamp delta. x [ncols][ldx] f32, y [ncols][ldy] f32, original rows. One launch for one column
- * (and two columns of short K), deterministic. The K-chunk partial rows, arrival counters and meeting slots live
+ * un-permute + clamp delta. x [ncols][ldx] f32, y [ncols][ldy] f32, original rows. One launch for one column; several
+ * columns on the matrix cores, with the activations quantized in that launch or (more than a block per wave) by one
+ * before it. Deterministic. The K-chunk partial rows, arrival counters and meeting slots live
  * in the tensor's handle: calls on one tensor from different streams must not overlap (on one stream they are
  * ordered); counters and slots are put back by each call. Records kernel launches only (capture-safe). */
 int p8x_mul_mat_vec(const p8x_tensor *t, const float *x, int ncols, size_t ldx, float *y, size_t ldy, void *stream);
-/* the same with the activation mode chosen: P8X_ACT_Q8_128 (as p8x_mul_mat_vec), P8X_ACT_Q8_1 (ggml block_q8_1 of x',
- * quantized inside the GEMV's launch, or by a prep launch within a graph evaluation, below), or P8X_ACT_X16 (1..4
- * columns: both planes of each column through one GEMV, summed, then the clamp delta; the reference's CPU default) */
+/* the same with the activation mode chosen: P8X_ACT_Q8_128 (as p8x_mul_mat_vec), P8X_ACT_Q8_1 (ggml block_q8_1 of x')
+ * or P8X_ACT_X16 (1..4 columns: both planes of each column as two columns of one GEMV, summed, then the clamp delta; the
+ * reference's CPU default); both quantize x as the several-column call above does */
 int p8x_mul_mat_vec_act(const p8x_tensor *t, int act, const float *x, int ncols, size_t ldx, float *y, size_t ldy, void *stream);
 /* Marks the start of a graph evaluation (ggml_vr_cpu_graph_begin, CPU.patch:1148). After the first call, a
  * p8x_mul_mat_vec_act call in P8X_ACT_X16 or P8X_ACT_Q8_1 mode reuses the activation that the previous such call on
@@ -158,10 +159,8 @@ int p8x_mul_mat_vec_multi(const p8x_tensor *const *tensors, int n, const float *
 int p8x_mul_mat_vec_glu(const p8x_tensor *gate, const p8x_tensor *up, const float *x, size_t ldx, float *out, void *stream);
 /* The two calls above with the activation mode chosen, as p8x_mul_mat_vec_act (the reference's CPU path defaults to
  * x16, CPU.patch:1157-1160, and prepares the activation once for consecutive mul_mats on the same input and c,
- * CPU.patch:1142-1143, :1171-1180): P8X_ACT_Q8_128 runs the one-launch forms above; P8X_ACT_X16 prepares x once in
- * tensor 0's (the gate's) workspace and runs each tensor's GEMV on it (both planes as two columns, summed, then the
- * clamp delta); P8X_ACT_Q8_1 runs each tensor's block_q8_1 GEMV with x quantized in its launch; then for the GLU
- * silu(gate) * up. Same values as p8x_mul_mat_vec_act per tensor. Calls sharing a tensor are ordered on one stream. */
+ * CPU.patch:1142-1143, :1171-1180): P8X_ACT_Q8_128 runs the one-launch forms above; P8X_ACT_X16 and P8X_ACT_Q8_1 run each
+ * tensor's p8x_mul_mat_vec_act call (which quantizes x itself); then for the GLU silu(gate) * up. Same values as p8x_mul_mat_vec_act per tensor. Calls sharing a tensor are ordered on one stream. */
 int p8x_mul_mat_vec_multi_act(const p8x_tensor *const *tensors, int n, int act, const float *x, size_t ldx, float *const *y,
                               const size_t *ldy, void *stream);
 int p8x_mul_mat_vec_glu_act(const p8x_tensor *gate, const p8x_tensor *up, int act, const float *x, size_t ldx, float *out, void *stream);

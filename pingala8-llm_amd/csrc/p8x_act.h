@@ -126,10 +126,7 @@ __device__ __forceinline__ void quantize_block_q8_128(const float *__restrict__ 
 // ggml block_q8_1 of one rotated 256-block (quantize_row_q8_1_ref convention): lane l holds values 4l..4l+3, so the
 // eight lanes 8i..8i+7 form 32-block i: d = max|x'| / 127 over it, q = round-half-away(x' / d), s = d * sum(q).
 // dd and s are the float values the block stores as fp16.
-__device__ __forceinline__ void quantize_block_q8_1(const float *__restrict__ x, const float *__restrict__ ic, int lane, uint32_t &packed,
-                                                    float &dd, float &s) {
-    BlockLane in;
-    in.load(x, ic, lane);
+__device__ __forceinline__ void quantize_loaded_q8_1(const BlockLane &in, int lane, uint32_t &packed, float &dd, float &s) {
     float v[4];
     rotate_block_lane(in, lane, v);
     float am = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
@@ -144,6 +141,33 @@ __device__ __forceinline__ void quantize_block_q8_1(const float *__restrict__ x,
     for (int m = 1; m < 8; m <<= 1) sum += __shfl_xor(sum, m);
     s = (float)sum * dd;
     packed = (uint32_t)(uint8_t)qi[0] | ((uint32_t)(uint8_t)qi[1] << 8) | ((uint32_t)(uint8_t)qi[2] << 16) | ((uint32_t)(uint8_t)qi[3] << 24);
+}
+
+__device__ __forceinline__ void quantize_block_q8_1(const float *__restrict__ x, const float *__restrict__ ic, int lane, uint32_t &packed,
+                                                    float &dd, float &s) {
+    BlockLane in;
+    in.load(x, ic, lane);
+    quantize_loaded_q8_1(in, lane, packed, dd, s);
+}
+
+// x16 planes of one 256-block (vrc_prep_block16, CPU.patch:575-616): d = max|x'| / 8191 per 128-column half, q =
+// round-half-even(x' / d) (14 bits), q = 128 hi + lo; lane l gets the packed int8 of elements 4l..4l+3 of each plane
+// and dd = d (the planes' scales are 128 d and d).
+__device__ __forceinline__ void quantize_loaded_x16(const BlockLane &in, int lane, uint32_t &ph, uint32_t &pl, float &dd) {
+    float v[4];
+    rotate_block_lane(in, lane, v);
+    float am = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    am = half_wave_max(am, lane);
+    dd = div_rn(am, 8191.f);
+    const float id = dd > 0.f ? div_rn(1.f, dd) : 0.f;
+    ph = pl = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int q = __float2int_rn(v[e] * id);
+        const int hi = (q + 64) >> 7, lo = q - 128 * hi;
+        ph |= (uint32_t)(uint8_t)hi << (8 * e);
+        pl |= (uint32_t)(uint8_t)lo << (8 * e);
+    }
 }
 
 }  // namespace p8x

@@ -87,19 +87,6 @@ __global__ __launch_bounds__(64) void k_act_x16(const float *__restrict__ x, siz
     (void)nsl;
 }
 
-// x16 products: y[n][ro] = (plane sums: hi column 2n + lo column 2n + 1, already in original rows) + the clamp delta
-// of row ro on the original activations, as the reference sums its two planes then adds the delta (CPU.patch:1193)
-__global__ __launch_bounds__(256) void k_x16_combine(const float *__restrict__ yv, int rows, const float *__restrict__ x, size_t ldx,
-                                                     const int *__restrict__ cp, const uint16_t *__restrict__ cc, const float *__restrict__ cv,
-                                                     float *__restrict__ y, size_t ldy) {
-    const int ro = blockIdx.x * 256 + threadIdx.x, n = blockIdx.y;
-    if (ro >= rows) return;
-    float v = yv[(size_t)(2 * n) * rows + ro] + yv[(size_t)(2 * n + 1) * rows + ro];
-    const float *xr = x + (size_t)n * ldx;
-    for (int e = cp[ro]; e < cp[ro + 1]; ++e) v += cv[e] * xr[cc[e]];
-    y[(size_t)n * ldy + ro] = v;
-}
-
 // out[r] = silu(g[r]) * u[r], silu(g) = g / (1 + e^-g) (ggml's swiglu): the gated input from two finished products
 __global__ __launch_bounds__(256) void k_glu_rows(const float *__restrict__ g, const float *__restrict__ u, int rows, float *__restrict__ out) {
     const int r = blockIdx.x * 256 + threadIdx.x;
@@ -232,9 +219,17 @@ int launch_gemv(const p8x_tensor *t, int act, const void *q, const float *d, int
                 float *y, size_t ldy, int32_t *partials, hipStream_t st) {
     const int cm = class_set(t->class_tiles, t->lin_words != 0);
     if (partials) return launch_gemv_range(t, act, q, d, ncols, x, ldx, y, ldy, partials, 0, t->ng, st);
-    // the row-group kernel: one column, or two columns of a one-class tensor with K <= 8192 (measured faster
-    // than the multi-column task kernel there, slower for longer K and more columns)
-    if (act == P8X_ACT_Q8_128 && !q && (ncols == 1 || (ncols == 2 && t->nb <= 32 && (cm == kCmC3 || cm == kCmC6)))) {
+    // x given: block_q8_1 and several columns run on the matrix cores, except two q8/128 columns where the dots are
+    // still faster (us a call, dots / matrix cores): class-3 tensors of few row groups and short K (1024 x 4096: 8.2 / 9.2;
+    // 4096 x 4096: 8.7 / 8.3 to 9.4), which the row-group kernel takes, and tensors of every class, whose tiles need more
+    // registers than the matrix-core kernel has at four waves per SIMD (4096 x 4096: 10.5 / 12.3), which the task kernel
+    // takes. From three columns the matrix cores win everywhere (4096 x 4096, class 3: 12.2 / 8.6 at three columns, 25.7
+    // / 9.5 at eight; block_q8_1: 9.6 / 7.9 at one column, 26.3 / 13.0 at six).
+    const bool two_rg = ncols == 2 && t->nb <= 32 && 2 * t->ng <= num_cus() && cm == kCmC3;
+    if (!q && (act == P8X_ACT_Q8_1 || (ncols > 1 && !two_rg && !(ncols == 2 && cm == kCmAll))))
+        return launch_gemv_mx(t, act, nullptr, nullptr, ncols, 1, x, ldx, y, ldy, st);
+    // the row-group kernel: one column, or two of a small class-3 tensor
+    if (act == P8X_ACT_Q8_128 && !q && (ncols == 1 || two_rg)) {
         // one linear, x quantized in the launch
         int kc;
         const int nks = rg_plan(t, ncols, &kc);
@@ -368,20 +363,9 @@ __global__ __launch_bounds__(256) void k_act_x16_batch(const ActJob *__restrict_
     const int b = gb - J.blk0;
     BlockLane in;
     in.load(J.x + (size_t)n * J.ldx + 256 * b, J.ic + 256 * b, lane);
-    float v[4];
-    rotate_block_lane(in, lane, v);
-    float am = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-    am = half_wave_max(am, lane);
-    const float dd = div_rn(am, 8191.f);
-    const float id = dd > 0.f ? div_rn(1.f, dd) : 0.f;
-    uint32_t ph = 0, pl = 0;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int q = __float2int_rn(v[e] * id);
-        const int hi = (q + 64) >> 7, lo = q - 128 * hi;
-        ph |= (uint32_t)(uint8_t)hi << (8 * e);
-        pl |= (uint32_t)(uint8_t)lo << (8 * e);
-    }
+    uint32_t ph, pl;
+    float dd;
+    quantize_loaded_x16(in, lane, ph, pl, dd);
     const int hs = lane >> 5, t = lane & 31;
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
@@ -808,25 +792,14 @@ int p8x_mul_mat_vec_multi(const p8x_tensor *const *tensors, int n, const float *
     return launch_gemv_multi(tensors, n, x, ldx, y, ldy, nullptr, (hipStream_t)stream);
 }
 
-// The shared-input calls with another activation mode. Q8_1: each tensor's block_q8_1 GEMV quantizes x in its own
-// launch (every tensor rotates its input the same way, so the blocks are the same); X16: the planes are prepared once
-// (in tensor 0's workspace) and each tensor multiplies them as two columns into its plane rows, then its combine
-// (planes summed, then the delta).
+// The shared-input calls with another activation mode: each tensor's call quantizes x itself (every tensor rotates its
+// input the same way, so the activations are the same).
 static int multi_act(const p8x_tensor *const *ts, int n, int act, const float *x, size_t ldx, float *const *y, const size_t *ldy, hipStream_t st) {
-    const p8x_tensor *t0 = ts[0];
     int rc;
-    if (act == P8X_ACT_Q8_1) {   // each GEMV's tasks quantize their chunks (the tensors share the rotation)
-        for (int i = 0; i < n; ++i)
-            if ((rc = launch_gemv(ts[i], P8X_ACT_Q8_1, nullptr, nullptr, 1, x, ldx, y[i], ldy[i], nullptr, st))) return rc;
-        return P8X_OK;
-    }
-    if ((rc = launch_act_x16(t0, x, 1, ldx, t0->wq, t0->wd, nullptr, t0->wq + t0->K, t0->wd + t0->nsl, nullptr, 2 * t0->K, st))) return rc;
     for (int i = 0; i < n; ++i) {
-        const p8x_tensor *t = ts[i];
-        if ((rc = launch_gemv(t, P8X_ACT_Q8_128, t0->wq, t0->wd, 2, nullptr, 0, t->wy, t->rows, nullptr, st))) return rc;
-        hipLaunchKernelGGL(k_x16_combine, dim3((t->rows + 255) / 256, 1), dim3(256), 0, st, (const float *)t->wy, t->rows, x, ldx,
-                           (const int *)t->cp, (const uint16_t *)t->cc, (const float *)t->cv, y[i], ldy[i]);
-        if ((rc = hip_check(hipGetLastError(), "k_x16_combine launch"))) return rc;
+        if (act == P8X_ACT_Q8_1) rc = launch_gemv_mx(ts[i], act, nullptr, nullptr, 1, 1, x, ldx, y[i], ldy[i], st);
+        else rc = launch_gemv_mx(ts[i], P8X_ACT_Q8_128, nullptr, nullptr, 1, 2, x, ldx, y[i], ldy[i], st);
+        if (rc) return rc;
     }
     return P8X_OK;
 }
@@ -895,24 +868,6 @@ int launch_act_x16(const p8x_tensor *t, const float *x, int ncols, size_t ldx, i
                    int32_t *sl, int qstride, hipStream_t st) {
     hipLaunchKernelGGL(k_act_x16, dim3(t->nb, ncols), dim3(64), 0, st, x, ldx, (const float *)t->ic, t->K, qh, dh, sh, ql, dl, sl, qstride);
     return hip_check(hipGetLastError(), "k_act_x16 launch");
-}
-
-// x16 products of ncols <= 4 columns: both planes of every column quantized into the handle's workspace as 2 ncols
-// virtual columns (hi of column n at 2n, lo at 2n + 1), one 8-bit-per-128 GEMV over them into the plane rows, then
-// the combine pass
-int launch_gemv_x16(const p8x_tensor *t, const float *x, int ncols, size_t ldx, float *y, size_t ldy, hipStream_t st) {
-    return launch_gemv_x16_on(t, x, ncols, ldx, y, ldy, t->wq, t->wd, false, st);
-}
-
-// the same with the planes' buffers given (q [2 ncols][K], d [2 ncols][nsl]); have: they already hold x's planes
-int launch_gemv_x16_on(const p8x_tensor *t, const float *x, int ncols, size_t ldx, float *y, size_t ldy, int8_t *q, float *d, bool have,
-                       hipStream_t st) {
-    int rc;
-    if (!have && (rc = launch_act_x16(t, x, ncols, ldx, q, d, nullptr, q + t->K, d + t->nsl, nullptr, 2 * t->K, st))) return rc;
-    if ((rc = launch_gemv(t, P8X_ACT_Q8_128, q, d, 2 * ncols, nullptr, 0, t->wy, t->rows, nullptr, st))) return rc;
-    hipLaunchKernelGGL(k_x16_combine, dim3((t->rows + 255) / 256, ncols), dim3(256), 0, st, (const float *)t->wy, t->rows, x, ldx,
-                       (const int *)t->cp, (const uint16_t *)t->cc, (const float *)t->cv, y, ldy);
-    return hip_check(hipGetLastError(), "k_x16_combine launch");
 }
 
 // ---------------------------------------------------------------------------------------- prepared-activation reuse

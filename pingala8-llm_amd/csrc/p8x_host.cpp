@@ -313,6 +313,8 @@ int p8x_prepare(const void *slot, size_t n, int rows, int K, int on_device, p8x_
             int kc;
             const int rn = rg_plan(t, nc, &kc);
             if (rn > 1) t->wpart_floats = std::max(t->wpart_floats, (size_t)rn * nc * rows);
+            for (int planes = 1; planes * nc <= P8X_MAX_COLS && planes <= 2; ++planes)
+                t->wpart_floats = std::max(t->wpart_floats, mx_part_floats(t, nc, planes));
             if (nc == 1) {
                 const GemvPlan pp = gemv_plan(t, 1, act, true);
                 if (pp.nks > 1) t->wpart_floats = std::max(t->wpart_floats, (size_t)pp.nks * rows);
@@ -468,22 +470,23 @@ int p8x_mul_mat_vec_act(const p8x_tensor *t, int act, const float *x, int ncols,
     int rc;
     if (act == P8X_ACT_Q8_128)   // one launch: every task quantizes its chunk of x itself (same arithmetic as the prep)
         return launch_gemv(t, act, nullptr, nullptr, ncols, x, ldx, y, ldy, nullptr, st);
-    // x16 and, within a graph evaluation (p8x_graph_begin), block_q8_1 prepare x in a launch of their own, and a later
+    // Within a graph evaluation (p8x_graph_begin) x16 and block_q8_1 prepare x in a launch of their own, and a later
     // call on the same input and rotation reuses the activation the previous call prepared (CPU.patch:1171-1180);
-    // outside one, block_q8_1 is quantized by the GEMV's tasks (one launch)
+    // outside one the GEMV quantizes x itself
     bool have = false;
     if (act == P8X_ACT_Q8_1) {
         uint8_t *blk = act_reuse(t, act, x, ncols, ldx, (size_t)36 * ncols * (t->K / 32), st, &have);
-        if (!blk) return launch_gemv(t, act, nullptr, nullptr, ncols, x, ldx, y, ldy, nullptr, st);
-        if (!have && (rc = launch_act_q8_1(t, x, ncols, ldx, blk, st))) return rc;
-        return launch_gemv(t, act, blk, nullptr, ncols, x, ldx, y, ldy, nullptr, st);
+        if (blk && !have && (rc = launch_act_q8_1(t, x, ncols, ldx, blk, st))) return rc;
+        return launch_gemv_mx(t, act, blk, nullptr, ncols, 1, x, ldx, y, ldy, st);
     }
     if (act == P8X_ACT_X16) {
         if (2 * ncols > P8X_MAX_COLS) return set_error(P8X_ERR_ARG, "p8x_mul_mat_vec: x16 takes at most %d columns", P8X_MAX_COLS / 2);
         const size_t qb = ((size_t)2 * ncols * t->K + 255) & ~(size_t)255;
         uint8_t *c = act_reuse(t, act, x, ncols, ldx, qb + (size_t)8 * ncols * t->nsl, st, &have);
-        if (!c) return launch_gemv_x16(t, x, ncols, ldx, y, ldy, st);
-        return launch_gemv_x16_on(t, x, ncols, ldx, y, ldy, reinterpret_cast<int8_t *>(c), reinterpret_cast<float *>(c + qb), have, st);
+        int8_t *q = reinterpret_cast<int8_t *>(c);
+        float *d = c ? reinterpret_cast<float *>(c + qb) : nullptr;
+        if (c && !have && (rc = launch_act_x16(t, x, ncols, ldx, q, d, nullptr, q + t->K, d + t->nsl, nullptr, 2 * t->K, st))) return rc;
+        return launch_gemv_mx(t, P8X_ACT_Q8_128, q, d, ncols, 2, x, ldx, y, ldy, st);
     }
     return set_error(P8X_ERR_ARG, "p8x_mul_mat_vec: act %d", act);
 }

@@ -83,9 +83,11 @@ int launch_act_q8_1(const p8x_tensor *t, const float *x, int ncols, size_t ldx, 
 // x16 planes: column n's hi plane at qh + n qstride, lo plane at ql + n qstride (scales and sums at n qstride / 128)
 int launch_act_x16(const p8x_tensor *t, const float *x, int ncols, size_t ldx, int8_t *qh, float *dh, int32_t *sh, int8_t *ql, float *dl,
                    int32_t *sl, int qstride, hipStream_t st);
-int launch_gemv_x16(const p8x_tensor *t, const float *x, int ncols, size_t ldx, float *y, size_t ldy, hipStream_t st);
-int launch_gemv_x16_on(const p8x_tensor *t, const float *x, int ncols, size_t ldx, float *y, size_t ldy, int8_t *q, float *d, bool have,
-                       hipStream_t st);
+// single call on the matrix cores (p8x_gemv_mx.hip): q (and d) prepared activations or null (x quantized by the call);
+// planes 2: x16. Its K-chunk partial rows: mx_part_floats of wpart.
+int launch_gemv_mx(const p8x_tensor *t, int act, const void *q, const float *d, int ncols, int planes, const float *x, size_t ldx, float *y, size_t ldy,
+                   hipStream_t st);
+size_t mx_part_floats(const p8x_tensor *t, int ncols, int planes);
 // Prepared-activation reuse within one graph evaluation (p8x_graph_begin): a device array of kActCacheBytes per GPU
 // holds the activation the last x16 / block_q8_1 call prepared; act_reuse returns it (nullptr: no reuse, use the
 // tensor's workspace) and whether it already holds this call's activation (same evaluation, input, stride, columns,
