@@ -616,6 +616,21 @@ int p8x_gemv_batch_create_ex(const p8x_tensor *const *tensors, const float *cons
                 const int nks = std::min(16, std::max(1, tensors[i]->nb / 2));
                 kcs[i] = (tensors[i]->nb + nks - 1) / nks;
             }
+        // A wave streams a unit's tiles one after another (~1.2 us each for mixed classes), so in a launch of a few layers
+        // one whole-K unit of the longest linear outlasts everything else. No unit is longer than 0.7 of the tiles a wave
+        // has on average: 5 / 2 layers of the Llama-3.1-8B linears (ffn_down 56 blocks, mixed) 86 / 74 -> 61 / 33 us, 2
+        // layers at 8 columns 152 -> 87 (0.5 and 1.0 of the average are within 5% of it, 0.25 5 to 20% slower); 16 layers,
+        // where the average exceeds the longest unit, keep their plan (189).
+        if (!small_launch) {
+            size_t tiles = 0;
+            for (int i = 0; i < njobs; ++i) tiles += tensors[i]->nt;
+            const int cap = std::max(2, (int)(7 * tiles / (10 * (size_t)launch_waves)));
+            for (int i = 0; i < njobs; ++i)
+                if (kcs[i] > cap) {
+                    const int nks = std::min(16, (tensors[i]->nb + cap - 1) / cap);
+                    kcs[i] = (tensors[i]->nb + nks - 1) / nks;
+                }
+        }
     }
     for (int i = 0; i < njobs; ++i) {
         const p8x_tensor *t = tensors[i];
