@@ -349,9 +349,10 @@ __device__ __forceinline__ void lo_read(uint32_t (&w)[8], const uint32_t *p, int
     }
 }
 
-// chunks 16 p .. 16 p + 15 of the lane-slice -> stage-2 ints, packed P[2 i] = (y0, y1), P[2 i + 1] = (y2, y3)
+// chunks 16 p .. 16 p + 15 of the lane-slice -> stage-2 ints, packed P[2 i] = (y0, y1), P[2 i + 1] = (y2, y3); returns
+// their coset bits (bit i = chunk 16 p + i)
 template <int C>
-__device__ __forceinline__ void lo_decode(const uint32_t (&w)[8], int d, int p16, const uint2 *tab4, uint32_t (&P)[32]) {
+__device__ __forceinline__ uint32_t lo_decode(const uint32_t (&w)[8], int d, int p16, const uint2 *tab4, uint32_t (&P)[32]) {
     constexpr int W1 = w1_of(C);
     uint32_t r[8], z;
     if constexpr (W1 == 8) {
@@ -388,6 +389,7 @@ __device__ __forceinline__ void lo_decode(const uint32_t (&w)[8], int d, int p16
         P[2 * i + 1] = e.y;
         if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // 4 lookups at a time
     }
+    return H;
 }
 
 template <int CM>
@@ -416,10 +418,11 @@ __device__ __forceinline__ void lo_read_any(int c, uint32_t (&w)[8], const uint3
     }
 }
 
-// butterflies h = 4, 8, 16, 32 of the lane's 64 values (exact int16)
+// butterflies h = 4 << M0 .. 4 << (M1 - 1) of the lane's 64 values (exact int16)
+template <int M0 = 0, int M1 = 4>
 __device__ __forceinline__ void lo_stages(uint32_t (&P)[32]) {
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
+    for (int m = M0; m < M1; ++m) {
         const int st = 1 << m;
 #pragma unroll
         for (int i = 0; i < 16; ++i)
@@ -596,6 +599,281 @@ __global__ __launch_bounds__(kLoThreads) __attribute__((amdgpu_waves_per_eu(4, 4
     }
 }
 
+// ------------------------------------------------------------------------------------------------ dequantize, classes 0-4 and 6
+// k_dequant_lo for tensors that also hold tiles of classes 4 and 6 (two stages, v = 4 (A[f1] + h c) + A[f2] + h c, so
+// |v| <= 510 while every |A[f] + h c| <= kLo46Max). Such a tile's integer stages stop earlier:
+//   * up to stage 8 (sums of 16 values: 16 * 510 * 2047 < 2^24) the reference's sums are exact and equal the integers
+//     times S; stage 16 is the integer butterfly and the one multiply by S (it adds two exact values: RN((I_a +- I_b) S));
+//   * stages 32, 64 and 128 are the reference's f32 additions on the reference's operands.
+// A tensor with a row scale that is not finite, a wider codebook or classes 5 or 7 goes through k_dequant. 4096 x 14336 to
+// fp16: the ffn_down mix (classes 2, 3 and 4) 60.7 -> 44.7 us a call, class 6 66.1 -> 52.0 against k_dequant (classes 0-3:
+// 33.4 in k_dequant_lo); 1024 x 4096 13.8 -> 13.0. Bound by the decode's VALU and the staging waits, as k_dequant_lo; it
+// needs 168 registers, three workgroups per CU.
+constexpr int kLo46Max = 102;
+constexpr int kLo46Per = 3;   // workgroups per CU (168 registers)
+__host__ __device__ constexpr int lo46_tile_words(int cm) { return (cm >> 6) & 1 ? 1024 : 768; }   // whole 256-word copies
+
+// stage 1 of any of the classes: words and chunks as in lo_read / lo_decode (classes 3, 4 and 6 hold the same 8-bit fields)
+template <int CM>
+__device__ __forceinline__ void lo46_read(int c, uint32_t (&w)[8], const uint32_t *p, int j, int d) {
+    switch (c) {
+        case 1: lo_read<1>(w, p, j, d); break;
+        case 2: lo_read<2>(w, p, j, d); break;
+        case 3: lo_read<3>(w, p, j, d); break;
+        case 4: lo_read<4>(w, p, j, d); break;
+        case 6: if constexpr ((CM >> 6) & 1) { lo_read<6>(w, p, j, d); break; } [[fallthrough]];
+        default:
+#pragma unroll
+            for (int i = 0; i < 8; ++i) w[i] = 0u;
+            break;
+    }
+}
+__device__ __forceinline__ uint32_t lo46_decode(int c, const uint32_t (&w)[8], int d, int p16, const uint2 *tab4, uint32_t (&P)[32]) {
+    switch (c) {
+        case 0:
+#pragma unroll
+            for (int i = 0; i < 32; ++i) P[i] = 0u;   // zero weights
+            return 0u;
+        case 1: return lo_decode<1>(w, d, p16, tab4, P);
+        case 2: return lo_decode<2>(w, d, p16, tab4, P);
+        default: return lo_decode<3>(w, d, p16, tab4, P);
+    }
+}
+
+// stage 2 of a class 4 / 6 lane-slice: its 16 fields from chunk 16 p on, as bytes (word i: fields 4 i .. 4 i + 3)
+template <int C>
+__device__ __forceinline__ void lo_read2(uint32_t (&w)[4], const uint32_t *p, int j, int p16) {
+    constexpr int W1 = w1_of(C), W2 = w2_of(C), NW = nw_of(C);
+    static_assert(W2 == 8 || W2 == 2, "classes 4 and 6");
+    if constexpr (W2 == 8) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = p[dev_word(W1 + i + (p16 >> 2), j, NW)];
+    } else {
+        w[0] = p[dev_word(W1 + (p16 >> 4), j, NW)];
+        w[1] = w[2] = w[3] = 0u;
+    }
+}
+
+// adds the second stage: P = 4 P + its table entries (the tile's coset bits H, bit i = chunk 16 p + i)
+template <int C>
+__device__ __forceinline__ void lo_add2(const uint32_t (&w)[4], uint32_t H, const uint2 *tab4, uint32_t (&P)[32]) {
+    const s16x2 four = {4, 4};
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const uint32_t f = C == 6 ? __builtin_amdgcn_ubfe(w[i >> 2], 8 * (i & 3), 8) : __builtin_amdgcn_ubfe(w[0], 2 * i, 2);
+        const uint2 e = tab4[(f << 1) | __builtin_amdgcn_ubfe(H, i, 1)];
+        P[2 * i] = as_u32(as_s16x2(P[2 * i]) * four + as_s16x2(e.x));
+        P[2 * i + 1] = as_u32(as_s16x2(P[2 * i + 1]) * four + as_s16x2(e.y));
+        if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// the wave's 64 16-byte pieces straight into LDS at dst (direct-to-LDS load)
+__device__ __forceinline__ void lds_copy16(const uint32_t *src, uint32_t *dst) {
+    __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
+}
+
+// f32 butterfly h = 64 across lanes j and j + 32: a + b in the lower (sg = 1), a - b in the upper (sg = -1)
+__device__ __forceinline__ float lo_cross64(float v, float sg) {
+    const auto pr = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    const float b = sg * __uint_as_float(pr[1]);
+    return __uint_as_float(pr[0]) + b;
+}
+
+template <int DT, int CM>
+__global__ __launch_bounds__(kLoThreads) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_dequant_lo46(const DecodeArgs a) {
+    static_assert(DT == P8X_F16 || DT == P8X_BF16, "16-bit outputs (f32 goes through k_dequant)");
+    __shared__ uint2 tab4[512];
+    __shared__ __align__(16) float icw[kLoWaves][256];
+    __shared__ __align__(16) uint32_t stg[kLoWaves][32 * kLoBandWords];   // one 32-row x 128-byte band per wave
+    constexpr int kLoTileWords = lo46_tile_words(CM);
+    __shared__ __align__(16) uint32_t pay[kLoWaves][kLoTileWords];         // the next tile's payload, per wave
+    const int tid = threadIdx.x, lane_in = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    for (int i = tid; i < 512; i += kLoThreads) tab4[i] = fwht4_entry(a.a2[(i & 1) * 256 + (i >> 1)]);
+    __syncthreads();
+    size_t first, last;
+    wg_range(a, first, last);
+    first += w;
+    if (first >= last) return;
+    LoNext nx;
+    // The next tile's payload is copied into the wave's LDS buffer (direct-to-LDS loads, no registers held) before
+    // this tile's output stores, and its tile word comes through the scalar cache: stores count in vmcnt like loads,
+    // so data requested after them could only be waited for together with them. A tile's row scale and row are
+    // loaded at the start of its own iteration and first used after its decode.
+    auto issue = [&](size_t q, int lane) {
+        int g, b;
+        tile_of(a, q, g, b);
+        g = __builtin_amdgcn_readfirstlane(g);
+        b = __builtin_amdgcn_readfirstlane(b);
+        const uint32_t mt = as_const(a.M)[(size_t)g * a.nb + b];
+        nx.c = (int)(mt >> 29);
+        const int chunks = 16 * nw_of(nx.c);   // 16-byte pieces of the tile (both half-slices)
+        if (chunks) {
+            const uint32_t *base = a.D + (mt & 0x1FFFFFFFu);
+#pragma unroll
+            for (int i = 0; i < (kLoTileWords + 255) / 256; ++i)   // lanes past the tile repeat its last piece
+                if (i < 2 || 64 * i < chunks) lds_copy16(base + 4 * min(64 * i + lane, chunks - 1), pay[w] + 256 * i);
+        }
+    };
+    int icb = -1;
+    issue(first, lane_in);
+    for (size_t q = first; q < last; q += kLoWaves) {
+        // lane-derived values formed per tile: held across the loop they would be spilled, and a spill reload waits
+        // for every memory operation in flight (this tile's stores included)
+        int lane = lane_in;
+        __asm__ volatile("" : "+v"(lane));
+        const int j = lane & 31, p = lane >> 5, p16 = 16 * p;
+        const int d = p16;
+        const s16x2 sg = {(short)(p ? -1 : 1), (short)(p ? -1 : 1)};
+        const int c = nx.c;
+        // this tile's copy is in LDS (the compiler does not order these reads behind the copies of lds_copy16)
+        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        uint32_t w0[8], w1[8], v0[4] = {}, v1[4] = {};
+        lo46_read<CM>(c, w0, pay[w], j, d);
+        lo46_read<CM>(c, w1, pay[w] + nw_of(c) * 32, j, d);
+        if constexpr ((CM >> 4) & 1)
+            if (c == 4) { lo_read2<4>(v0, pay[w], j, p16); lo_read2<4>(v1, pay[w] + nw_of(4) * 32, j, p16); }
+        if constexpr ((CM >> 6) & 1)
+            if (c == 6) { lo_read2<6>(v0, pay[w], j, p16); lo_read2<6>(v1, pay[w] + nw_of(6) * 32, j, p16); }
+        __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read before the next tile's copy overwrites it
+        int g, b;
+        tile_of(a, q, g, b);
+        g = __builtin_amdgcn_readfirstlane(g);
+        b = __builtin_amdgcn_readfirstlane(b);
+        const uint16_t s16 = a.S[(size_t)b * a.rows + 32 * g + j];
+        const int rof = a.prmd[32 * g + j], ro = rof & 0x7FFF;
+        if (q + kLoWaves < last) issue(q + kLoWaves, lane);
+        // one half-slice at a time through its integer stages (only its 32 packed registers are being built)
+        uint32_t P0[32], P1[32];
+        const bool hi = c > 3;   // wave-uniform
+        auto half_ints = [&](const uint32_t (&wh)[8], const uint32_t (&vh)[4], uint32_t (&P)[32]) {
+            const uint32_t H = lo46_decode(c, wh, d, p16, tab4, P);
+            if constexpr ((CM >> 4) & 1)
+                if (c == 4) lo_add2<4>(vh, H, tab4, P);
+            if constexpr ((CM >> 6) & 1)
+                if (c == 6) lo_add2<6>(vh, H, tab4, P);
+            lo_stages<0, 3>(P);
+            if (!hi) {
+                lo_stages<3, 4>(P);
+                lo_stage64(P, sg);
+            }
+            __asm__ volatile("" ::: "memory");
+        };
+        half_ints(w0, v0, P0);
+        half_ints(w1, v1, P1);
+        const float S = half_to_float(s16);
+        if (b != icb) {   // this block's ic / 16 into the wave's row (wave-local)
+            const float4 c4 = reinterpret_cast<const float4 *>(a.ic + 256 * b)[lane];
+            reinterpret_cast<float4 *>(icw[w])[lane] = make_float4(c4.x * 0.0625f, c4.y * 0.0625f, c4.z * 0.0625f, c4.w * 0.0625f);
+            icb = b;
+        }
+        int e0 = 0, e1 = 0;
+        if (rof & 0x8000) { e0 = a.cp[ro]; e1 = a.cp[ro + 1]; }
+        const bool deltas = __builtin_amdgcn_ballot_w64(e0 < e1) != 0;   // wave-uniform
+        const float *icl = icw[w] + 64 * p;
+        // the packed 16-bit outputs: OUT[h][g] holds values 8 g .. 8 g + 7 of half-slice h (columns 64 p + ..)
+        uint32_t OUT[2][8][4];
+        // clamp delta (original row, column) in entry order, then the packed outputs of values 2 k4 .. 2 k4 + 7
+        auto emit = [&](int k4, float (&o)[2][8]) {
+            if (deltas) {
+                for (int e = e0; e < e1; ++e) {
+                    const int col = (int)a.cc[e] - 256 * b;
+                    const float dv = a.cv[e];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+#pragma unroll
+                        for (int i = 0; i < 8; ++i)
+                            if (col == 128 * h + 64 * p + 2 * k4 + i) o[h][i] += dv;
+                }
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int q2 = 0; q2 < 4; ++q2) {
+                    if constexpr (DT == P8X_F16) {   // v_cvt_pk_f16_f32: both RNE
+                        const f16x2 hv = {(_Float16)o[h][2 * q2], (_Float16)o[h][2 * q2 + 1]};
+                        OUT[h][k4 >> 2][q2] = __builtin_bit_cast(uint32_t, hv);
+                    } else {                          // v_cvt_pk_bf16_f32: both RNE
+                        const bf16x2 hv = {(__bf16)o[h][2 * q2], (__bf16)o[h][2 * q2 + 1]};
+                        OUT[h][k4 >> 2][q2] = __builtin_bit_cast(uint32_t, hv);
+                    }
+                    pin(OUT[h][k4 >> 2][q2]);
+                }
+            __builtin_amdgcn_sched_barrier(0);   // one group at a time: its packed ints are consumed as its outputs appear
+        };
+        // stage 128 (the two half-slices), * ic / 16
+        auto last = [&](int k, int kk, float x0, float x1, float y0, float y1, float (&o)[2][8]) {
+            const float2 c0 = *reinterpret_cast<const float2 *>(icl + 2 * k);
+            const float2 c1 = *reinterpret_cast<const float2 *>(icl + 128 + 2 * k);
+            o[0][2 * kk] = (x0 + y0) * c0.x;
+            o[0][2 * kk + 1] = (x1 + y1) * c0.y;
+            o[1][2 * kk] = (x0 - y0) * c1.x;
+            o[1][2 * kk + 1] = (x1 - y1) * c1.y;
+        };
+        if (!hi) {
+#pragma unroll
+            for (int k4 = 0; k4 < 32; k4 += 4) {
+                float o[2][8];
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) {
+                    const s16x2 x = as_s16x2(P0[k4 + kk]), y = as_s16x2(P1[k4 + kk]);
+                    last(k4 + kk, kk, (float)x.x * S, (float)x.y * S, (float)y.x * S, (float)y.y * S, o);
+                }
+                emit(k4, o);
+            }
+        } else {
+            const float sgf = p ? -1.f : 1.f;
+            // stage 32 (packed values k and k + 16 of the lane), stage 64
+#pragma unroll
+            for (int k4 = 0; k4 < 16; k4 += 4) {
+                float o[2][2][8];
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) {
+                    const int k = k4 + kk;
+                    float t[2][2][2];   // [stage-32 output: k, k + 16][half][value]
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const s16x2 x = as_s16x2(h ? P1[k] : P0[k]), y = as_s16x2(h ? P1[k + 16] : P0[k + 16]);
+                        const float a0 = (float)x.x * S, a1 = (float)x.y * S, b0 = (float)y.x * S, b1 = (float)y.y * S;
+                        t[0][h][0] = lo_cross64(a0 + b0, sgf);
+                        t[0][h][1] = lo_cross64(a1 + b1, sgf);
+                        t[1][h][0] = lo_cross64(a0 - b0, sgf);
+                        t[1][h][1] = lo_cross64(a1 - b1, sgf);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) last(k + 16 * u, kk, t[u][0][0], t[u][0][1], t[u][1][0], t[u][1][1], o[u]);
+                }
+                emit(k4, o[0]);
+                emit(k4 + 16, o[1]);
+            }
+        }
+        // Out through the wave's LDS band, one (half-slice, quarter) band of the tile at a time: the lanes that own
+        // it write their 128 bytes, then each store instruction covers 8 rows x 128 bytes (whole lines).
+        uint32_t *sw = stg[w];
+        int orows[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) orows[i] = (__shfl(rof, 8 * i + (lane >> 3)) & 0x7FFF) - a.row0;   // row of piece 64 i + lane
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int qq = 0; qq < 2; ++qq) {
+                if (p == qq)
+#pragma unroll
+                    for (int gg = 0; gg < 8; ++gg)
+                        *reinterpret_cast<uint4 *>(sw + j * kLoBandWords + 4 * gg) = make_uint4(OUT[h][gg][0], OUT[h][gg][1], OUT[h][gg][2], OUT[h][gg][3]);
+                __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the band is written
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int row = 8 * i + (lane >> 3), piece = lane & 7;
+                    const uint4 val = *reinterpret_cast<const uint4 *>(sw + row * kLoBandWords + 4 * piece);
+                    if ((unsigned)orows[i] < (unsigned)a.nrows)
+                        *reinterpret_cast<uint4 *>((uint16_t *)a.out + (size_t)orows[i] * a.ld + 256 * b + 128 * h + 64 * qq + 8 * piece) = val;
+                }
+                __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read before the next band overwrites it
+            }
+    }
+}
+
 static DecodeArgs decode_args(const p8x_tensor *t, void *out, size_t ld) {
     DecodeArgs a{};
     a.M = t->M; a.S = t->S; a.D = t->D; a.a2 = t->a2; a.prm = t->prm; a.prmd = t->prmd;
@@ -617,16 +895,34 @@ static bool only_class3(const p8x_tensor *t) {
     return true;
 }
 
-// every tile of class 0-3: the integer-butterfly dequantizer
-static bool classes_upto3(const p8x_tensor *t) {
-    for (int c = 4; c < 8; ++c) if (t->class_tiles[c]) return false;
-    return true;
+constexpr int kLo46 = (1 << 4) | (1 << 6);
+// every tile of class 0-3, or also 4 and 6 with a codebook and scales that keep the integer stages exact: the
+// integer-butterfly dequantizer; *cm = its class set
+static bool lo_classes(const p8x_tensor *t, int *cm) {
+    *cm = 0;
+    for (int c = 1; c < 8; ++c) if (t->class_tiles[c]) *cm |= 1 << c;
+    if (*cm & ((1 << 5) | (1 << 7))) return false;
+    if (!(*cm & kLo46)) return true;
+    // a wave takes a tile in about 8 us however few there are, k_dequant a little less (256 x 512: 13.2 and 12.7 us)
+    if (t->nt < (size_t)num_cus()) return false;
+    for (int i = 0; i < 512; ++i)
+        for (int e = 0; e < 4; ++e) {
+            const int v = (int8_t)(t->a2_host[i] >> (8 * e));
+            if (v > kLo46Max || v < -kLo46Max) return false;
+        }
+    return t->scales_finite;
 }
 
 template <int CM>
 static void launch_deq_lo(int dtype, const DecodeArgs &a, int grid, hipStream_t st) {
     if (dtype == P8X_F16) hipLaunchKernelGGL((k_dequant_lo<P8X_F16, CM>), dim3(grid), dim3(kLoThreads), 0, st, a);
     else hipLaunchKernelGGL((k_dequant_lo<P8X_BF16, CM>), dim3(grid), dim3(kLoThreads), 0, st, a);
+}
+
+template <int CM>
+static void launch_deq_lo46(int dtype, const DecodeArgs &a, int grid, hipStream_t st) {
+    if (dtype == P8X_F16) hipLaunchKernelGGL((k_dequant_lo46<P8X_F16, CM>), dim3(grid), dim3(kLoThreads), 0, st, a);
+    else hipLaunchKernelGGL((k_dequant_lo46<P8X_BF16, CM>), dim3(grid), dim3(kLoThreads), 0, st, a);
 }
 
 template <int CM>
@@ -664,10 +960,14 @@ int launch_dequant(const p8x_tensor *t, int dtype, int row0, int nrows, void *ou
         }
         a.g0 = lo; a.gn = hi - lo + 1; a.nt = (size_t)a.gn * a.bn;
     }
-    if (classes_upto3(t) && dtype != P8X_F32) {
-        const int grid = (int)std::min<size_t>((a.nt + kLoWaves - 1) / kLoWaves, (size_t)num_cus() * 4);
+    int cm;
+    if (dtype != P8X_F32 && lo_classes(t, &cm)) {
+        constexpr int kLo = (1 << 1) | (1 << 2) | (1 << 3);
+        const int grid = (int)std::min<size_t>((a.nt + kLoWaves - 1) / kLoWaves, (size_t)num_cus() * (cm & kLo46 ? kLo46Per : 4));
         if (only_class3(t)) launch_deq_lo<(1 << 3)>(dtype, a, grid, st);
-        else launch_deq_lo<(1 << 1) | (1 << 2) | (1 << 3)>(dtype, a, grid, st);
+        else if (!(cm & kLo46)) launch_deq_lo<kLo>(dtype, a, grid, st);
+        else if (!((cm >> 6) & 1)) launch_deq_lo46<kLo | (1 << 4)>(dtype, a, grid, st);
+        else launch_deq_lo46<kLo | kLo46>(dtype, a, grid, st);
     } else if (only_class3(t)) {
         launch_deq<(1 << 3)>(t, dtype, a, st);
     } else {

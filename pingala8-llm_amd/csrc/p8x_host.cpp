@@ -53,12 +53,15 @@ void side_offsets(size_t n, size_t rows, size_t K, size_t nd, size_t off[6]) {
 }
 
 // row scales [nb][rows] -> [ng][nb][32], one element per thread
-__global__ void k_regroup_scales(const uint16_t *__restrict__ S, uint16_t *__restrict__ Sg, int nb, int rows, size_t n) {
+// bad (or null): set to 1 if a scale is infinite or NaN
+__global__ void k_regroup_scales(const uint16_t *__restrict__ S, uint16_t *__restrict__ Sg, int nb, int rows, size_t n, unsigned *bad) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const size_t gb = i >> 5;
     const int j = (int)(i & 31), g = (int)(gb / nb), b = (int)(gb % nb);
-    Sg[i] = S[(size_t)b * rows + 32 * g + j];
+    const uint16_t s = S[(size_t)b * rows + 32 * g + j];
+    Sg[i] = s;
+    if (bad && (s & 0x7C00u) == 0x7C00u) *bad = 1u;   // every writer stores the same word
 }
 
 // Field k of a region of W-bit fields starting at word o of a lane's words (bit string little-endian across words).
@@ -322,8 +325,6 @@ int p8x_prepare(const void *slot, size_t n, int rows, int K, int on_device, p8x_
         }
     }
     if ((rc = alloc((void **)&t->Sg, 64 * nt, "regrouped scales"))) return fail(rc);
-    hipLaunchKernelGGL(k_regroup_scales, dim3((unsigned)((32 * nt + 255) / 256)), dim3(256), 0, 0, t->S, t->Sg, nb, rows, 32 * nt);
-    if ((rc = hip_check(hipGetLastError(), "p8x_prepare: regroup scales"))) return fail(rc);
     if ((rc = alloc((void **)&t->a2, 512 * 4 + 512 * 8, "tables"))) return fail(rc);
     if ((rc = alloc((void **)&t->ic, 4 * (size_t)K, "ic"))) return fail(rc);
     if ((rc = alloc((void **)&t->cp, 4 * (size_t)(rows + 1), "delta rows"))) return fail(rc);
@@ -371,6 +372,16 @@ int p8x_prepare(const void *slot, size_t n, int rows, int K, int on_device, p8x_
         if ((rc = hip_check(hipMemcpy(t->cv, cv.data(), 4 * (size_t)nd, hipMemcpyHostToDevice), "p8x_prepare: csr"))) return fail(rc);
     }
     if ((rc = hip_check(hipMemset(t->wcnt, 0, 4 * (size_t)ng), "p8x_prepare: counters"))) return fail(rc);
+    const bool check_scales = t->class_tiles[4] || t->class_tiles[6];   // the counters' first word holds the answer
+    hipLaunchKernelGGL(k_regroup_scales, dim3((unsigned)((32 * nt + 255) / 256)), dim3(256), 0, 0, t->S, t->Sg, nb, rows, 32 * nt,
+                       check_scales ? t->wcnt : (unsigned *)nullptr);
+    if ((rc = hip_check(hipGetLastError(), "p8x_prepare: regroup scales"))) return fail(rc);
+    if (check_scales) {
+        unsigned bad = 0;
+        if ((rc = hip_check(hipMemcpy(&bad, t->wcnt, 4, hipMemcpyDeviceToHost), "p8x_prepare: scales"))) return fail(rc);
+        t->scales_finite = bad == 0;
+        if (bad && (rc = hip_check(hipMemset(t->wcnt, 0, 4), "p8x_prepare: counters"))) return fail(rc);
+    }
     if ((rc = upload_job(t))) return fail(rc);
     if ((rc = hip_check(hipDeviceSynchronize(), "p8x_prepare: sync"))) return fail(rc);
     *out = t;
