@@ -224,6 +224,163 @@ __device__ __forceinline__ void gemv_tile_quad(const TaskCtx<NCOL, P8X_ACT_Q8_12
     for (int n = 0; n < NCOL; ++n) yacc[n] += ((float)isum[n] * sm.xd[n * NSC + 2 * bl + c.hs]) * sc;
 }
 
+// A tile whose class is known at run time only, one of the class set CM (loaded as AnyQuads): every stage's fields are
+// brought to bytes (the narrow ones; most are bytes as loaded), then one body per number of stages serves every class.
+// A body per class keeps so many registers in reach that a prefetched tile spills, and the spill reloads wait for the
+// prefetch (28 to 85 spilled registers at 128; none this way).
+template <int CM>
+struct ByteFields {
+    static constexpr int NST = (CM >> 7) & 1 ? 3 : (CM >> 4) & 7 ? 2 : 1;   // most stages of the set
+    static constexpr int NQ = (CM >> 7) & 1 ? 6 : (CM >> 6) & 1 ? 4 : (CM >> 5) & 1 ? 3 : 2;   // 16-byte groups of its largest class
+    uint32_t f[NST][8];   // [stage][i]: fields 4 i .. 4 i + 3
+    uint32_t H;           // coset bits
+
+    template <int C>
+    __device__ __forceinline__ void expand(const AnyQuads<NQ> &t) {
+        if constexpr ((CM >> C) & 1) {
+            constexpr int W1 = w1_of(C), W2 = w2_of(C);
+            const QuadSlice<C> r = t.template as<C>();
+            if constexpr (W1 < 8)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    uint32_t v = 0;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int k = 4 * i + e;
+                        v |= (field_at<W1 - 1, QuadSlice<C>::O1>(r.w, k) | (__builtin_amdgcn_ubfe(r.w[0], k, 1) << (W1 - 1))) << (8 * e);
+                    }
+                    f[0][i] = v;
+                }
+            if constexpr (W2 > 0 && W2 < 8)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    uint32_t v = 0;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v |= field_at<W2, QuadSlice<C>::O2>(r.w, 4 * i + e) << (8 * e);
+                    f[1][i] = v;
+                }
+        }
+    }
+    // c is wave-uniform, in CM
+    __device__ __forceinline__ void from(const AnyQuads<NQ> &t, uint32_t c) {
+#pragma unroll
+        for (int s = 0; s < NST; ++s)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[s][i] = 8 * s + i < 4 * NQ ? t.w[8 * s + i < 4 * NQ ? 8 * s + i : 0] : 0u;
+        switch (c) {
+            case 1: expand<1>(t); break;
+            case 2: expand<2>(t); break;
+            case 4: expand<4>(t); break;
+            case 5: expand<5>(t); break;
+            default: break;   // 3, 6, 7: bytes as loaded
+        }
+        H = trellis_coset_bits(c < 3u ? t.w[0] : labels_from_bytes(f[0]));   // classes 1 and 2 store the labels in word 0
+    }
+};
+
+// Dots of NST stages over one pass of the activation words: the stages' sums, shifted (2^SH of the class), added
+template <int NST, int CM, int NCOL, int XW>
+__device__ __forceinline__ void byte_dots(const uint32_t *tab, const ByteFields<CM> &b, uint32_t bankbytes, lds_cptr xl, int sh1, int (&isum)[NCOL]) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    int acc[NST][NCOL];
+#pragma unroll
+    for (int s = 0; s < NST; ++s)
+#pragma unroll
+        for (int n = 0; n < NCOL; ++n) acc[s][n] = 0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        u32x4 xv[NCOL];
+#pragma unroll
+        for (int n = 0; n < NCOL; ++n) xv[n] = *reinterpret_cast<const __attribute__((address_space(3))) u32x4 *>(xl + n * XW + 4 * q);
+        const uint32_t hq = coset_bytes(b.H, bankbytes, q);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            uint32_t w[NST];
+#pragma unroll
+            for (int s = 0; s < NST; ++s) w[s] = lds_word(tab, __builtin_amdgcn_perm(b.f[s][q], hq, 0x0c0c0000u | ((4u + e) << 8) | e));
+#pragma unroll
+            for (int n = 0; n < NCOL; ++n)
+#pragma unroll
+                for (int s = 0; s < NST; ++s) acc[s][n] = __builtin_amdgcn_sdot4((int)w[s], (int)xv[n][e], acc[s][n], false);
+        }
+        __asm__ volatile("" ::: "memory");   // one group of 4 chunks at a time: bounds the live registers
+    }
+#pragma unroll
+    for (int n = 0; n < NCOL; ++n) {
+        isum[n] = acc[0][n];
+        if constexpr (NST == 2) isum[n] = (acc[0][n] << sh1) + acc[1][n];
+        if constexpr (NST == 3) isum[n] = acc[0][n] * (1 << sh1_of(7)) + acc[1][n] * (1 << sh2_of(7)) + acc[2][n];
+    }
+}
+
+// The wave's tiles of a tensor of mixed classes, blocks b0 .. b1 - 1 of its row groups: the next tile always in flight
+// (through the prep, through the tile before it and across row groups), and the tile word after it, which its load needs.
+// A set of one class (tiles in order, none of class 0) computes its payload offsets and reads no tile words.
+// What it measured against runs of one class at a time (a body and a prefetch per class, each run's first tile waited for):
+// 14336 x 4096 of class 6 14.2 -> 9.6 us, of all classes 21.1 -> 10.7; 4096 x 14336 of classes 2-4 13.1 -> 10.4; q, k, v of a
+// 4096-wide layer (v class 6) 9.0 -> 7.4. Class 3 alone keeps GemvRun (deeper prefetch, no expansion): 14336 x 4096 in
+// 7.6 us against 8.4 this way.
+template <int CM>
+struct AnyRun {
+    static constexpr int ONE = CM == kCmC6 ? 6 : 0;
+    AnyQuads<ByteFields<CM>::NQ> nxt;
+    uint32_t cls;         // of nxt
+    uint32_t mt, ti;      // word and index of the tile after nxt
+    int g, b, b0, b1, gadd;   // its place; row groups step by gadd
+
+    // past the tensor: one of its last tiles, loaded and never used
+    __device__ __forceinline__ void word(const GemvJob &J) {
+        ti = (uint32_t)min(g, J.ng - 1) * (uint32_t)J.nb + (uint32_t)min(b, J.nb - 1);
+        if constexpr (!ONE) mt = as_const(J.M)[ti];
+        const bool last = b + 1 == b1;
+        g += last ? gadd : 0;
+        b = last ? b0 : b + 1;
+    }
+    template <int NCOL>
+    __device__ __forceinline__ void issue(const TaskCtx<NCOL, P8X_ACT_Q8_128> &c) {
+        const GemvJob &J = *c.J;
+        cls = ONE ? (uint32_t)ONE : mt >> 29;
+        __builtin_amdgcn_s_setprio(2);   // loads issued at raised priority (see wave_run)
+        nxt.load(buffer_rsrc(J.D, J.dbytes), ONE ? ti * (uint32_t)(4 * 64 * nw_of(ONE)) : (mt & 0x1FFFFFFFu) * 4u, ONE ? (uint32_t)nw_of(ONE) : nw_run(cls),
+                 c.hs, c.j, buffer_rsrc(J.S, (uint32_t)J.nb * J.rows * 2u), ti * 64u, 2u * c.j);
+        __builtin_amdgcn_s_setprio(0);
+        word(J);
+    }
+    template <int NCOL>
+    __device__ __forceinline__ void begin(const TaskCtx<NCOL, P8X_ACT_Q8_128> &c, int gfirst, int gadd_, int b0_, int b1_) {
+        g = gfirst; b = b0 = b0_; b1 = b1_; gadd = gadd_;
+        word(*c.J);
+        issue<NCOL>(c);
+    }
+    // the next n tiles (all of a row group's, first block b0) into yacc
+    template <int NCOL, typename SM>
+    __device__ __forceinline__ void run(const TaskCtx<NCOL, P8X_ACT_Q8_128> &c, const SM &sm, int n, float (&yacc)[NCOL]) {
+        for (int i = 0; i < n; ++i) {
+            AnyQuads<ByteFields<CM>::NQ> t = nxt;
+            const uint32_t cl = cls;
+            issue<NCOL>(c);
+            __asm__ volatile("" ::: "memory");
+            pin(t.w);
+            pin(t.p);
+            pin(t.s);
+            if (!ONE && cl == 0u) continue;   // zero weights
+            const int bl = b0 + i - c.b0;
+            lds_cptr xl = (lds_cptr)(sm.xq + bl * 128 + c.xlane);
+            __asm__ volatile("" : "+v"(xl));
+            ByteFields<CM> f;
+            f.from(t, cl);
+            int isum[NCOL];
+            if (ByteFields<CM>::NST == 3 && cl == 7u) byte_dots<ByteFields<CM>::NST, CM, NCOL, SM::kXW>(sm.tab, f, c.bankbytes, xl, 0, isum);
+            else if (cl > 3u) byte_dots<2, CM, NCOL, SM::kXW>(sm.tab, f, c.bankbytes, xl, cl == 5u ? sh1_of(5) : sh1_of(4), isum);
+            else byte_dots<1, CM, NCOL, SM::kXW>(sm.tab, f, c.bankbytes, xl, 0, isum);
+            const float sc = half_to_float(t.s);
+#pragma unroll
+            for (int k = 0; k < NCOL; ++k) yacc[k] += ((float)isum[k] * sm.xd[k * SM::kNSC + 2 * bl + c.hs]) * sc;
+        }
+    }
+};
+static_assert(sh1_of(4) == sh1_of(6), "classes 4 and 6 share a shift");
+
 // A run of consecutive tiles of class C in row group g: the run's extent is found from the tile words
 // first, then NBUF register buffers rotate so that NBUF - 1 following tiles are in flight while the current
 // one is decoded. Every step issues its prefetch (past the run's end through an empty resource, which reads
@@ -690,8 +847,8 @@ void k_gemv_rg(RgJobs jobs, const uint32_t *__restrict__ a2, int gc_) {
     int b0 = c.b0 + wk * per + min(wk, rem), b1 = b0 + per + (wk < rem ? 1 : 0);   // the wave's K range
     if (team >= gc) b1 = b0;
     // Loads in the order their data is needed (vector loads return in order): the wave's activation blocks, the
-    // codebook words of the table; then, for a one-class tensor, the wave's first run of tiles (its first row group
-    // over its K range), whose payload stays in flight while the table is written and x is quantized.
+    // codebook words of the table; then the wave's first tiles (class 3: its first run, other sets: its first tile), whose
+    // payload stays in flight while the table is written and x is quantized.
     BlockLane in[RQ];
 #pragma unroll
     for (int i = 0; i < RQ; ++i) {
@@ -705,19 +862,21 @@ void k_gemv_rg(RgJobs jobs, const uint32_t *__restrict__ a2, int gc_) {
     P8X_STAMP(1);
     CosetTableFill<64 * WAVES> fill;
     fill.load(a2, tid);
-    constexpr int PC = CM == kCmC3 ? 3 : CM == kCmC6 ? 6 : 0;
-    GemvRun<NCOL, P8X_ACT_Q8_128, false, PC ? PC : 3, gemv_nbuf(NCOL, PC ? PC : 3), true> pre;
+    constexpr bool RUN3 = CM == kCmC3;   // class 3 alone: runs of tiles as their class; else tile by tile (AnyRun)
+    GemvRun<NCOL, P8X_ACT_Q8_128, false, 3, gemv_nbuf(NCOL, 3), true> pre;
     const int gstep = nwg / nks;
     const int gfirst = wgl / nks + min(team, gc - 1) * gstep;
-    const bool pre_on = PC != 0 && team < gc && gfirst < J.ng && b0 < b1;
+    const bool pre_on = RUN3 && team < gc && gfirst < J.ng && b0 < b1;
+    AnyRun<CM> any;
     __asm__ volatile("" ::: "memory");
-    if constexpr (PC != 0) {
+    if constexpr (RUN3) {
         // on every path (a wave without work requests one in-range tile it never reads), so that no control-flow
         // merge before the table stores makes the compiler wait for these loads there
         c.g = min(gfirst, J.ng - 1);
         const int bb = pre_on ? b0 : min(b0, J.nb - 1);
         pre.begin(c, bb, pre_on ? b1 : bb + 1);
     }
+    if constexpr (!RUN3) any.template begin<NCOL>(c, gfirst, gstep * gc, b0, b1);
     __asm__ volatile("" ::: "memory");
 #ifdef P8X_TIMELINE
     __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -745,26 +904,15 @@ void k_gemv_rg(RgJobs jobs, const uint32_t *__restrict__ a2, int gc_) {
         float yacc[NCOL];
 #pragma unroll
         for (int n = 0; n < NCOL; ++n) yacc[n] = 0.f;
-        int bstart = b0;
-        if (PC != 0 && first && pre_on) bstart = pre.finish(c, sm, yacc);   // the run begun before the prep
-        first = false;
-        for (int b = bstart; b < (g < J.ng ? b1 : b0);) {
-            if constexpr (PC != 0) {   // one class: no tile word to read
-                b = gemv_run<NCOL, P8X_ACT_Q8_128, false, PC, gemv_nbuf(NCOL, PC), true>(c, sm, b, b1, yacc);
-                continue;
-            }
-            const uint32_t mt = as_const(JB.M)[(size_t)g * JB.nb + b];
-            switch (mt >> 29) {
-                case 1: if constexpr ((CM >> 1) & 1) { b = gemv_run<NCOL, P8X_ACT_Q8_128, false, 1, gemv_nbuf(NCOL, 1), CM == (1 << 1)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                case 2: if constexpr ((CM >> 2) & 1) { b = gemv_run<NCOL, P8X_ACT_Q8_128, false, 2, gemv_nbuf(NCOL, 2), CM == (1 << 2)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                case 3: if constexpr ((CM >> 3) & 1) { b = gemv_run<NCOL, P8X_ACT_Q8_128, false, 3, gemv_nbuf(NCOL, 3), CM == (1 << 3)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                case 4: if constexpr ((CM >> 4) & 1) { b = gemv_run<NCOL, P8X_ACT_Q8_128, false, 4, gemv_nbuf(NCOL, 4), CM == (1 << 4)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                case 5: if constexpr ((CM >> 5) & 1) { b = gemv_run<NCOL, P8X_ACT_Q8_128, false, 5, gemv_nbuf(NCOL, 5), CM == (1 << 5)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                case 6: if constexpr ((CM >> 6) & 1) { b = gemv_run<NCOL, P8X_ACT_Q8_128, false, 6, gemv_nbuf(NCOL, 6), CM == (1 << 6)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                case 7: if constexpr ((CM >> 7) & 1) { b = gemv_run<NCOL, P8X_ACT_Q8_128, false, 7, gemv_nbuf(NCOL, 7), CM == (1 << 7)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                default: ++b; break;   // class 0: zero weights
-            }
+        const int bend = g < J.ng ? b1 : b0;
+        if constexpr (RUN3) {
+            int b = b0;
+            if (first && pre_on) b = pre.finish(c, sm, yacc);   // the run begun before the prep
+            while (b < bend) b = gemv_run<NCOL, P8X_ACT_Q8_128, false, 3, gemv_nbuf(NCOL, 3), true>(c, sm, b, b1, yacc);
+        } else {
+            any.run(c, sm, bend - b0, yacc);
         }
+        first = false;
         P8X_STAMP(5);
 #pragma unroll
         for (int n = 0; n < NCOL; ++n) {

@@ -7,8 +7,8 @@ namespace p8x {
 // several linears on one activation vector (one column): the MULTI instantiations
 int launch_gemv_rg_multi(int cm, const RgJobs &jobs, int ng, const uint32_t *a2, hipStream_t st) {
     if (cm == kCmC3) return launch_gemv_rg_t<kCmC3, 1, true>(jobs, ng, a2, st);
-    if (cm == kCmC6) return launch_gemv_rg_t<kCmC6, 1, true>(jobs, ng, a2, st);
     if (cm == kCmC234) return launch_gemv_rg_t<kCmC234, 1, true>(jobs, ng, a2, st);
+    if (cm == kCmC6) return launch_gemv_rg_t<kCmC6, 1, true>(jobs, ng, a2, st);
     if (cm == kCmC2346) return launch_gemv_rg_t<kCmC2346, 1, true>(jobs, ng, a2, st);
     return launch_gemv_rg_t<kCmAll, 1, true>(jobs, ng, a2, st);
 }

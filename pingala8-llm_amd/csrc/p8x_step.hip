@@ -112,7 +112,7 @@ __device__ __forceinline__ void step_stage(kptr<const StepStage> sp, int v, RgSm
     const int per = nbk / wpg, rem = nbk % wpg;
     int b0 = c.b0 + wk * per + min(wk, rem), b1 = b0 + per + (wk < rem ? 1 : 0);   // the wave's K range
     if (team >= gc) b1 = b0;
-    // the wave's activation blocks (agent-coherent loads), then, for a one-class chain, its first run of tiles
+    // the wave's activation blocks (agent-coherent loads), then its first tiles
     BlockLane in[RQ];
     const uint32_t xbytes = 4u * (uint32_t)J.K;
 #pragma unroll
@@ -132,16 +132,19 @@ __device__ __forceinline__ void step_stage(kptr<const StepStage> sp, int v, RgSm
         rec[6] |= min(__builtin_amdgcn_s_memrealtime() - rec[0], (u64)0xFFFF) << 16;
     }
 #endif
-    constexpr int PC = CM == kCmC3 ? 3 : CM == kCmC6 ? 6 : 0;
-    GemvRun<1, P8X_ACT_Q8_128, false, PC ? PC : 3, gemv_nbuf(1, PC ? PC : 3), true> pre;
+    constexpr bool RUN3 = CM == kCmC3;   // as in k_gemv_rg
+    GemvRun<1, P8X_ACT_Q8_128, false, 3, gemv_nbuf(1, 3), true> pre;
+    AnyRun<CM> any;
     const int gstep = nwg / nks;
     const int gfirst = wgl / nks + min(team, gc - 1) * gstep;
-    const bool pre_on = PC != 0 && team < gc && gfirst < J.ng && b0 < b1;
+    const bool pre_on = RUN3 && team < gc && gfirst < J.ng && b0 < b1;
     __asm__ volatile("" ::: "memory");
-    if constexpr (PC != 0) {   // on every path, as in k_gemv_rg
+    if constexpr (RUN3) {   // on every path, as in k_gemv_rg
         c.g = min(gfirst, J.ng - 1);
         const int bb = pre_on ? b0 : min(b0, J.nb - 1);
         pre.begin(c, bb, pre_on ? b1 : bb + 1);
+    } else {
+        any.template begin<1>(c, gfirst, gstep * gc, b0, b1);
     }
     __asm__ volatile("" ::: "memory");
 #ifdef P8X_TIMELINE
@@ -175,26 +178,15 @@ __device__ __forceinline__ void step_stage(kptr<const StepStage> sp, int v, RgSm
         int ro = 0;
         if (lead && lane < 32) ro = as_global(J.prmd)[32 * g + lane];
         float yacc[1] = {0.f};
-        int bstart = b0;
-        if (PC != 0 && first && pre_on) bstart = pre.finish(c, sm, yacc);
-        first = false;
-        for (int b = bstart; b < (g < J.ng ? b1 : b0);) {
-            if constexpr (PC != 0) {   // one class: no tile word to read
-                b = gemv_run<1, P8X_ACT_Q8_128, false, PC, gemv_nbuf(1, PC), true>(c, sm, b, b1, yacc);
-                continue;
-            }
-            const uint32_t mt = as_const(J.M)[(size_t)g * J.nb + b];
-            switch (mt >> 29) {
-                case 1: if constexpr ((CM >> 1) & 1) { b = gemv_run<1, P8X_ACT_Q8_128, false, 1, gemv_nbuf(1, 1), CM == (1 << 1)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                case 2: if constexpr ((CM >> 2) & 1) { b = gemv_run<1, P8X_ACT_Q8_128, false, 2, gemv_nbuf(1, 2), CM == (1 << 2)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                case 3: if constexpr ((CM >> 3) & 1) { b = gemv_run<1, P8X_ACT_Q8_128, false, 3, gemv_nbuf(1, 3), CM == (1 << 3)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                case 4: if constexpr ((CM >> 4) & 1) { b = gemv_run<1, P8X_ACT_Q8_128, false, 4, gemv_nbuf(1, 4), CM == (1 << 4)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                case 5: if constexpr ((CM >> 5) & 1) { b = gemv_run<1, P8X_ACT_Q8_128, false, 5, gemv_nbuf(1, 5), CM == (1 << 5)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                case 6: if constexpr ((CM >> 6) & 1) { b = gemv_run<1, P8X_ACT_Q8_128, false, 6, gemv_nbuf(1, 6), CM == (1 << 6)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                case 7: if constexpr ((CM >> 7) & 1) { b = gemv_run<1, P8X_ACT_Q8_128, false, 7, gemv_nbuf(1, 7), CM == (1 << 7)>(c, sm, b, b1, yacc); break; } [[fallthrough]];
-                default: ++b; break;   // class 0: zero weights
-            }
+        const int bend = g < J.ng ? b1 : b0;
+        if constexpr (RUN3) {
+            int b = b0;
+            if (first && pre_on) b = pre.finish(c, sm, yacc);
+            while (b < bend) b = gemv_run<1, P8X_ACT_Q8_128, false, 3, gemv_nbuf(1, 3), true>(c, sm, b, b1, yacc);
+        } else {
+            any.run(c, sm, bend - b0, yacc);
         }
+        first = false;
         yacc[0] += __shfl_xor(yacc[0], 32);
 #ifdef P8X_TIMELINE
         if (rec && round0 && tid == 0) rec[7] |= min(__builtin_amdgcn_s_memrealtime() - tin, (u64)0xFFFF) << 16;
