@@ -555,7 +555,11 @@ static MmPlan mm_plan(const p8x_tensor *t, int N) {
     // plan (and returns the same bits) as p8x_mul_mat wherever it runs at all
     const size_t xb = ((size_t)N * t->K * sizeof(_Float16) + 255) & ~(size_t)255;
     const size_t cap = xb < (size_t)P8X_NOALLOC_SCRATCH_BYTES ? (size_t)P8X_NOALLOC_SCRATCH_BYTES - xb : 0;
+#ifdef P8X_TIMELINE
+    MmPlan best{0, false, 4, 0, 0, 1, t->nb};   // the timeline build stamps k_mm's phases: k_mm at every token count
+#else
     MmPlan best{mm_rg_tiles(t, N), false, 4, 0, 0, 1, t->nb};
+#endif
     if (best.rg) return best;
     double best_cost = -1.0;
     auto consider = [&](bool dense, int nti, double block_us, double pro_us, double extra_us) {
@@ -573,8 +577,6 @@ static MmPlan mm_plan(const p8x_tensor *t, int N) {
     // at 256 x 128 (its decode needs the registers; 7.4 with the released ffn_down mix of classes 2, 3 and 4).
     if (c3) consider(false, 8, 7.5, 3.7, 0.0);
     consider(false, 4, c3 ? 3.9 : 7.4, c3 ? 3.7 : 5.0, 0.0);
-    // Decoded operands: a launch that writes 16 KB per tile (33 us for 117 MB), then 0.9 us per 32 tokens and block with
-    // every CU busy. 4096 x 14336, the ffn_down mix, 1500 tokens: k_mm 427 us a call, 276 here (two K ranges, 192-token
     // Decoded operands: a launch that writes 16 KB per tile (33 us for 117 MB), then 0.9 us per 32 tokens and block with
     // every CU busy. 4096 x 14336, the ffn_down mix, 1500 tokens: k_mm 443 us a call, 237 here (two K ranges, 192-token
     // tiles; the dense kernel alone 1.07 PFLOP/s, the card's library product 1.2). Class 3 keeps k_mm, whose decode is

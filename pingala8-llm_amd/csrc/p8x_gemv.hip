@@ -839,9 +839,9 @@ int p8x_mul_mat_vec_glu_act(const p8x_tensor *gate, const p8x_tensor *up, int ac
     int rc;
     if ((rc = check_shared_input(ts, 2, x, ldx, "p8x_mul_mat_vec_glu_act"))) return rc;
     if (gate->rows != up->rows) return set_error(P8X_ERR_ARG, "p8x_mul_mat_vec_glu_act: gate has %d rows, up %d", gate->rows, up->rows);
-    // the two products in original rows in each tensor's plane rows past the x16 planes (row block 2), then the gate
+    // the two products in original rows in each tensor's row workspace, then the gate
     hipStream_t st = (hipStream_t)stream;
-    float *const ys[2] = {gate->wy + 2 * (size_t)gate->rows, up->wy + 2 * (size_t)up->rows};
+    float *const ys[2] = {gate->wy, up->wy};
     const size_t ldys[2] = {(size_t)gate->rows, (size_t)up->rows};
     if ((rc = multi_act(ts, 2, act, x, ldx, ys, ldys, st))) return rc;
     hipLaunchKernelGGL(k_glu_rows, dim3((gate->rows + 255) / 256), dim3(256), 0, st, (const float *)ys[0], (const float *)ys[1], gate->rows, out);

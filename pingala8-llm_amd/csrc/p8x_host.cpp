@@ -335,7 +335,7 @@ int p8x_prepare(const void *slot, size_t n, int rows, int K, int on_device, p8x_
     if ((rc = alloc((void **)&t->wsum, 4 * (size_t)P8X_MAX_COLS * nsl, "sum"))) return fail(rc);
     if ((rc = alloc((void **)&t->wq81, (size_t)36 * P8X_MAX_COLS * (K / 32), "q8_1"))) return fail(rc);
     if ((rc = alloc((void **)&t->wpart, 4 * t->wpart_floats, "partials"))) return fail(rc);
-    if ((rc = alloc((void **)&t->wy, 4 * (size_t)P8X_MAX_COLS * rows, "x16 plane rows"))) return fail(rc);
+    if ((rc = alloc((void **)&t->wy, 4 * (size_t)rows, "swiglu rows"))) return fail(rc);
     if ((rc = alloc((void **)&t->wglu, 8 * (size_t)rows, "gate / up slots"))) return fail(rc);
     if ((rc = hip_check(hipMemset(t->wglu, 0, 8 * (size_t)rows), "p8x_prepare: gate / up slots"))) return fail(rc);
     if ((rc = alloc((void **)&t->wslot, 8 * (size_t)rows, "K-half slots"))) return fail(rc);

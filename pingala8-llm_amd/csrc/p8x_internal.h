@@ -44,7 +44,7 @@ struct p8x_tensor {
     float *wd = nullptr;             // [P8X_MAX_COLS][nsl]
     int32_t *wsum = nullptr;         // [P8X_MAX_COLS][nsl]
     uint8_t *wq81 = nullptr;         // block_q8_1 [P8X_MAX_COLS][K / 32]
-    float *wy = nullptr;             // x16 products: plane rows [2 x 4][rows]
+    float *wy = nullptr;             // x16 and block_q8_1 swiglu calls: the tensor's product [rows]
     unsigned lin_words = 0;               // one class, tiles in order: payload words per tile (else 0)
     unsigned long long *wglu = nullptr;   // gate / up meeting slots (this tensor as the gate) [rows], 0 between calls
     unsigned long long *wslot = nullptr;  // K-half meeting slots of one-column two-chunk plans [rows], 0 between calls
