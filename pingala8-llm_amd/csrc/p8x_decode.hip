@@ -605,7 +605,8 @@ __global__ __launch_bounds__(kLoThreads) __attribute__((amdgpu_waves_per_eu(4, 4
 //   * up to stage 8 (sums of 16 values: 16 * 510 * 2047 < 2^24) the reference's sums are exact and equal the integers
 //     times S; stage 16 is the integer butterfly and the one multiply by S (it adds two exact values: RN((I_a +- I_b) S));
 //   * stages 32, 64 and 128 are the reference's f32 additions on the reference's operands.
-// A tensor with a row scale that is not finite, a wider codebook or classes 5 or 7 goes through k_dequant. 4096 x 14336 to
+// A tensor with a row scale that is not finite or is negative (an integer sum of 0 times it is -0, the reference's sum of
+// scaled values that cancel is +0), a wider codebook or classes 5 or 7 goes through k_dequant. 4096 x 14336 to
 // fp16: the ffn_down mix (classes 2, 3 and 4) 60.7 -> 44.7 us a call, class 6 66.1 -> 52.0 against k_dequant (classes 0-3:
 // 33.4 in k_dequant_lo); 1024 x 4096 13.8 -> 13.0. Bound by the decode's VALU and the staging waits, as k_dequant_lo; it
 // needs 168 registers, three workgroups per CU.
@@ -910,7 +911,7 @@ static bool lo_classes(const p8x_tensor *t, int *cm) {
             const int v = (int8_t)(t->a2_host[i] >> (8 * e));
             if (v > kLo46Max || v < -kLo46Max) return false;
         }
-    return t->scales_finite;
+    return t->scales_plain;
 }
 
 template <int CM>

@@ -65,3 +65,35 @@ def test_dequant_lo46_infinite_scale(bad):
     H = t.dequantize(p8x.F16)
     nan = np.isnan(W)
     assert np.array_equal(np.isnan(H.view(np.float16)), nan) and np.array_equal(H[~nan], rne(W, p8x.F16)[~nan])
+
+
+@pytest.mark.parametrize("mix", ["c4", "c6", "c012346"])
+def test_dequant_lo46_negative_scales(mix):
+    """negative row scales over constant tiles: 255 of 256 rotated sums cancel, and the zeros keep the sign that the f32
+    dequantize gives them (-0 only where every term is -0)"""
+    rows, K = 1024, 2048
+    slot = p8x.synth_random(7, rows, K, class_p=MIXES[mix], nd=0).copy()
+    nt = rows // 32 * (K // 256)
+    M = slot[2064:2064 + 4 * nt].view(np.uint32)
+    doff = (2064 + 68 * nt + 15) // 16 * 16
+    slot[doff:doff + 256 * int(np.array((0, 4, 6, 8, 10, 12, 16, 24))[M >> 29].sum())] = 0
+    s = scales(slot, rows, K)
+    s[s != 0] |= 0x8000
+    W = O.Oracle(slot, rows, K).dequant()
+    assert (W == 0).any()
+    t = p8x.Tensor(slot, rows, K)
+    for dtype in (p8x.F16, p8x.BF16):
+        assert np.array_equal(t.dequantize(dtype), rne(W, dtype))
+
+
+def test_dequant_lo46_extreme_positive_scales():
+    """the extreme scales without the negative one, which would send the tensor to the general kernel"""
+    rows, K = 1024, 2048
+    slot = p8x.synth_random(5, rows, K, class_p=MIXES["c012346"], nd=6).copy()
+    s = scales(slot, rows, K)
+    nz = np.nonzero(s)[0]
+    s[nz] = np.random.default_rng(1).choice(np.array([0x7BFF, 0x1FFF, 0x03FF, 0x0001, 0x3FFF, 0x2AAB], np.uint16), nz.size)
+    W = O.Oracle(slot, rows, K).dequant()
+    t = p8x.Tensor(slot, rows, K)
+    for dtype in (p8x.F16, p8x.BF16):
+        assert np.array_equal(t.dequantize(dtype), rne(W, dtype))
