@@ -307,6 +307,8 @@ __global__ __launch_bounds__(kDecThreads) __attribute__((amdgpu_waves_per_eu(2, 
 //     butterfly (|I| <= 16384) followed by the one f32 multiply by S;
 //   * stage 128, * 0.0625 * ic (0.0625 folded into ic: scaling by a power of two is exact) and the clamp delta are
 //     the reference's f32 operations on the reference's operands; f16 / bf16 are the RNE conversions of that f32.
+// A tensor with a row scale that is not finite or is negative goes through k_dequant: an integer sum of 0 times such a
+// scale is NaN or -0, where the reference's sum of scaled values that cancel is not.
 // Lane (j, p) of a wave holds row j of the tile, columns 64 p .. 64 p + 63 of both half-slices: stages 4-32 stay in
 // the lane, stage 64 pairs lane j with lane j + 32 (v_permlane32_swap on the packed ints), stage 128 pairs the lane's
 // two half-slices. Each lane then writes 128 contiguous bytes (f16) per half-slice of its output row.
@@ -605,8 +607,7 @@ __global__ __launch_bounds__(kLoThreads) __attribute__((amdgpu_waves_per_eu(4, 4
 //   * up to stage 8 (sums of 16 values: 16 * 510 * 2047 < 2^24) the reference's sums are exact and equal the integers
 //     times S; stage 16 is the integer butterfly and the one multiply by S (it adds two exact values: RN((I_a +- I_b) S));
 //   * stages 32, 64 and 128 are the reference's f32 additions on the reference's operands.
-// A tensor with a row scale that is not finite or is negative (an integer sum of 0 times it is -0, the reference's sum of
-// scaled values that cancel is +0), a wider codebook or classes 5 or 7 goes through k_dequant. 4096 x 14336 to
+// A tensor with such a scale, a wider codebook or classes 5 or 7 goes through k_dequant. 4096 x 14336 to
 // fp16: the ffn_down mix (classes 2, 3 and 4) 60.7 -> 44.7 us a call, class 6 66.1 -> 52.0 against k_dequant (classes 0-3:
 // 33.4 in k_dequant_lo); 1024 x 4096 13.8 -> 13.0. Bound by the decode's VALU and the staging waits, as k_dequant_lo; it
 // needs 168 registers, three workgroups per CU.
@@ -902,7 +903,7 @@ constexpr int kLo46 = (1 << 4) | (1 << 6);
 static bool lo_classes(const p8x_tensor *t, int *cm) {
     *cm = 0;
     for (int c = 1; c < 8; ++c) if (t->class_tiles[c]) *cm |= 1 << c;
-    if (*cm & ((1 << 5) | (1 << 7))) return false;
+    if ((*cm & ((1 << 5) | (1 << 7))) || !t->scales_plain) return false;
     if (!(*cm & kLo46)) return true;
     // a wave takes a tile in about 8 us however few there are, k_dequant a little less (256 x 512: 13.2 and 12.7 us)
     if (t->nt < (size_t)num_cus()) return false;
@@ -911,7 +912,7 @@ static bool lo_classes(const p8x_tensor *t, int *cm) {
             const int v = (int8_t)(t->a2_host[i] >> (8 * e));
             if (v > kLo46Max || v < -kLo46Max) return false;
         }
-    return t->scales_plain;
+    return true;
 }
 
 template <int CM>

@@ -53,7 +53,7 @@ void side_offsets(size_t n, size_t rows, size_t K, size_t nd, size_t off[6]) {
 }
 
 // row scales [nb][rows] -> [ng][nb][32], one element per thread
-// bad (or null): set to 1 if a scale is infinite, NaN or has its sign bit set
+// bad: set to 1 if a scale is infinite, NaN or has its sign bit set
 __global__ void k_regroup_scales(const uint16_t *__restrict__ S, uint16_t *__restrict__ Sg, int nb, int rows, size_t n, unsigned *bad) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -61,7 +61,7 @@ __global__ void k_regroup_scales(const uint16_t *__restrict__ S, uint16_t *__res
     const int j = (int)(i & 31), g = (int)(gb / nb), b = (int)(gb % nb);
     const uint16_t s = S[(size_t)b * rows + 32 * g + j];
     Sg[i] = s;
-    if (bad && s >= 0x7C00u) *bad = 1u;   // every writer stores the same word
+    if (s >= 0x7C00u) *bad = 1u;   // every writer stores the same word
 }
 
 // Field k of a region of W-bit fields starting at word o of a lane's words (bit string little-endian across words).
@@ -372,16 +372,13 @@ int p8x_prepare(const void *slot, size_t n, int rows, int K, int on_device, p8x_
         if ((rc = hip_check(hipMemcpy(t->cv, cv.data(), 4 * (size_t)nd, hipMemcpyHostToDevice), "p8x_prepare: csr"))) return fail(rc);
     }
     if ((rc = hip_check(hipMemset(t->wcnt, 0, 4 * (size_t)ng), "p8x_prepare: counters"))) return fail(rc);
-    const bool check_scales = t->class_tiles[4] || t->class_tiles[6];   // the counters' first word holds the answer
-    hipLaunchKernelGGL(k_regroup_scales, dim3((unsigned)((32 * nt + 255) / 256)), dim3(256), 0, 0, t->S, t->Sg, nb, rows, 32 * nt,
-                       check_scales ? t->wcnt : (unsigned *)nullptr);
+    // the scale check's answer comes back in the counters' first word
+    hipLaunchKernelGGL(k_regroup_scales, dim3((unsigned)((32 * nt + 255) / 256)), dim3(256), 0, 0, t->S, t->Sg, nb, rows, 32 * nt, t->wcnt);
     if ((rc = hip_check(hipGetLastError(), "p8x_prepare: regroup scales"))) return fail(rc);
-    if (check_scales) {
-        unsigned bad = 0;
-        if ((rc = hip_check(hipMemcpy(&bad, t->wcnt, 4, hipMemcpyDeviceToHost), "p8x_prepare: scales"))) return fail(rc);
-        t->scales_plain = bad == 0;
-        if (bad && (rc = hip_check(hipMemset(t->wcnt, 0, 4), "p8x_prepare: counters"))) return fail(rc);
-    }
+    unsigned bad = 0;
+    if ((rc = hip_check(hipMemcpy(&bad, t->wcnt, 4, hipMemcpyDeviceToHost), "p8x_prepare: scales"))) return fail(rc);
+    t->scales_plain = bad == 0;
+    if (bad && (rc = hip_check(hipMemset(t->wcnt, 0, 4), "p8x_prepare: counters"))) return fail(rc);
     if ((rc = upload_job(t))) return fail(rc);
     if ((rc = hip_check(hipDeviceSynchronize(), "p8x_prepare: sync"))) return fail(rc);
     *out = t;

@@ -67,12 +67,13 @@ def test_dequant_lo46_infinite_scale(bad):
     assert np.array_equal(np.isnan(H.view(np.float16)), nan) and np.array_equal(H[~nan], rne(W, p8x.F16)[~nan])
 
 
-@pytest.mark.parametrize("mix", ["c4", "c6", "c012346"])
+@pytest.mark.parametrize("mix", ["c1", "c3", "c4", "c6", "c012346"])   # also classes 0-3 alone (k_dequant_lo's)
 def test_dequant_lo46_negative_scales(mix):
     """negative row scales over constant tiles: 255 of 256 rotated sums cancel, and the zeros keep the sign that the f32
     dequantize gives them (-0 only where every term is -0)"""
     rows, K = 1024, 2048
-    slot = p8x.synth_random(7, rows, K, class_p=MIXES[mix], nd=0).copy()
+    p = {"c1": (0, 1, 0, 0, 0, 0, 0, 0), "c3": (0, 0, 0, 1, 0, 0, 0, 0)}.get(mix) or MIXES[mix]
+    slot = p8x.synth_random(7, rows, K, class_p=p, nd=0).copy()
     nt = rows // 32 * (K // 256)
     M = slot[2064:2064 + 4 * nt].view(np.uint32)
     doff = (2064 + 68 * nt + 15) // 16 * 16
@@ -97,3 +98,16 @@ def test_dequant_lo46_extreme_positive_scales():
     t = p8x.Tensor(slot, rows, K)
     for dtype in (p8x.F16, p8x.BF16):
         assert np.array_equal(t.dequantize(dtype), rne(W, dtype))
+
+
+def test_dequant_classes_0_to_3_infinite_scale():
+    rows, K = 256, 2048
+    slot = p8x.synth_random(6, rows, K, class_p=(0, 1, 1, 1, 0, 0, 0, 0), nd=2).copy()
+    s = scales(slot, rows, K)
+    s[np.nonzero(s)[0][[3, 400]]] = 0x7C00
+    t = p8x.Tensor(slot, rows, K)
+    W = t.dequantize(p8x.F32)
+    H = t.dequantize(p8x.F16)
+    nan = np.isnan(W)
+    assert nan.any()
+    assert np.array_equal(np.isnan(H.view(np.float16)), nan) and np.array_equal(H[~nan], rne(W, p8x.F16)[~nan])
