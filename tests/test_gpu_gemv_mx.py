@@ -1,6 +1,8 @@
 """Single calls on the matrix cores (several q8/128 columns, x16, block_q8_1) against the oracle's fp64 GEMV of the same
 quantized activations, at the edges of the launch: one row group, more row groups than CUs (teams of waves), K in
 one block, K in counted and in paired chunks, quantized in the launch and before it."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -62,3 +64,25 @@ def test_gemv_mx_padded_strides():
     Y = y.to_numpy(np.float32, (n, ldy))
     assert (Y[:, rows:] == 7.0).all()
     assert np.array_equal(Y[:, :rows], t.mul_mat_vec(np.ascontiguousarray(X[:, :K])))
+
+
+@pytest.mark.parametrize("act,n", [("x16", 2), ("q81", 2), ("q8", 3)])
+def test_gemv_mx_strides_past_32_bits(act, n):
+    """columns 2^32 + 64 (three columns: 2^31 + 64) elements apart"""
+    rows, K, ld = 288, 1024, 1 << 32 if n == 2 else 1 << 31
+    ld += 64   # a stride cut to 32 bits would land inside the buffers
+    t = p8x.Tensor(p8x.synth_random(1, rows, K, class_p=MIX, nd=6), rows, K)
+    X = np.random.default_rng(n).standard_normal((n, K)).astype(np.float32)
+    ref = t.mul_mat_vec(X, act=ACT[act][0])
+    x, y = p8x.DeviceBuffer(4 * ((n - 1) * ld + K)), p8x.DeviceBuffer(4 * ((n - 1) * ld + rows))
+
+    def copy(dst, src, nbytes, kind):
+        p8x.hip_check(p8x.hip().hipMemcpy(ctypes.c_void_p(dst), ctypes.c_void_p(src), nbytes, kind), "hipMemcpy")
+    for c in range(n):
+        copy(x.ptr.value + 4 * c * ld, X[c].ctypes.data, 4 * K, p8x.H2D)
+    t.mul_mat_vec_dev(x, y, ncols=n, ldx=ld, ldy=ld, act=ACT[act][0])
+    p8x.synchronize()
+    Y = np.empty((n, rows), np.float32)
+    for c in range(n):
+        copy(Y[c].ctypes.data, y.ptr.value + 4 * c * ld, 4 * rows, p8x.D2H)
+    assert np.array_equal(Y, ref)
