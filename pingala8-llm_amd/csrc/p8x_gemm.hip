@@ -27,6 +27,7 @@
 #include "p8x_act.h"
 #include "p8x_lane.h"
 #include "p8x_mm.h"
+#include "p8x_operands.h"
 
 namespace p8x {
 
@@ -527,10 +528,20 @@ static int grow(void **p, size_t *have, size_t need, const char *what) {
         *p = nullptr;
         *have = 0;
     }
-    if (hipMalloc(p, need) != hipSuccess) return set_error(P8X_ERR_NOMEM, "%s: hipMalloc %zu bytes", what, need);
+    if (hipMalloc(p, need) != hipSuccess) {
+        (void)hipGetLastError();   // or the next launch's check would report it
+        return set_error(P8X_ERR_NOMEM, "%s: hipMalloc %zu bytes", what, need);
+    }
     *have = need;
     return P8X_OK;
 }
+
+struct HipApi {   // p8x_operands.h
+    static bool alloc(void **p, size_t n) { return hipMalloc(p, n) == hipSuccess; }
+    static void release(void *p) { (void)hipFree(p); }
+    static bool synchronize() { return hipDeviceSynchronize() == hipSuccess; }
+    static void clear_error() { (void)hipGetLastError(); }
+};
 
 struct MmPlan {
     int rg;    // 32-token tiles of the row-group GEMM (p8x_mm_rg.hip), which writes y itself; 0: k_mm, below
@@ -609,7 +620,7 @@ int reserve_mul_mat(const p8x_tensor *t, int n_max) {
     int rc;
     if ((rc = grow((void **)&tw->wx16, &tw->wx16_elems, xb, "p8x_mul_mat_reserve: activation workspace"))) return rc;
     if (planes && (rc = grow((void **)&tw->wmm, &tw->wmm_bytes, planes, "p8x_mul_mat_reserve: output planes"))) return rc;
-    if (wb && (rc = grow(&tw->wbw, &tw->wbw_bytes, wb, "p8x_mul_mat_reserve: decoded weights"))) return rc;
+    if (wb) (void)try_grow<HipApi>(&tw->wbw, &tw->wbw_bytes, wb);   // calls run k_mm without them
     return P8X_OK;
 }
 
@@ -692,10 +703,10 @@ int launch_mul_mat(const p8x_tensor *t, const void *x, int x_dtype, int N, size_
     size_t xb, pb, wb;
     mm_workspace(t, N, &xb, &pb, &wb);
     int rc;
-    if (wb && (rc = grow(&tw->wbw, &tw->wbw_bytes, wb, "p8x_mul_mat: decoded weights"))) return rc;
     if ((rc = grow((void **)&tw->wx16, &tw->wx16_elems, xb, "p8x_mul_mat: activation workspace"))) return rc;
     if (pb && (rc = grow((void **)&tw->wmm, &tw->wmm_bytes, pb, "p8x_mul_mat: output planes"))) return rc;
-    return launch_mul_mat_ws(t, x, x_dtype, N, ldx, y, ldy, reinterpret_cast<_Float16 *>(tw->wx16), tw->wmm, wb ? tw->wbw : nullptr, st);
+    return launch_mul_mat_ws(t, x, x_dtype, N, ldx, y, ldy, reinterpret_cast<_Float16 *>(tw->wx16), tw->wmm,
+                             wb && try_grow<HipApi>(&tw->wbw, &tw->wbw_bytes, wb) ? tw->wbw : nullptr, st);
 }
 
 // ------------------------------------------------------------------------------------------------ no-allocation variant
