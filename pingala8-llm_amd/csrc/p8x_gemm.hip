@@ -453,15 +453,22 @@ void k_mm(MmJob J) {
 }
 #undef P8X_MM_LAP
 
+// The kernels before this one on the stream have ended (the shared operand buffer, p8x_operands.h). A null word: no mark.
+__device__ __forceinline__ void set_mark(const OperandMark &m) {
+    if (m.word && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(m.word, m.n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__global__ __launch_bounds__(64) void k_mm_mark(OperandMark m) { set_mark(m); }   // calls without k_mm_finish
+
 // y[n][ro] = sum over K splits (split order) of the sorted planes at row pinv[ro], plus the clamp delta on the
 // original activations. One workgroup per token: the planes are read coalesced into LDS (sorted order), the
 // un-permute gathers from LDS, the stores are coalesced.
 template <typename XT>
 __global__ __launch_bounds__(1024) void k_mm_finish(const float *__restrict__ ws, int nsplit, int N, int rows, const int16_t *__restrict__ pinv,
                                                     const int *__restrict__ cp, const uint16_t *__restrict__ cc, const float *__restrict__ cv,
-                                                    const XT *__restrict__ x, size_t ldx, float *__restrict__ y, size_t ldy) {
+                                                    const XT *__restrict__ x, size_t ldx, float *__restrict__ y, size_t ldy, OperandMark mark) {
     extern __shared__ __attribute__((aligned(16))) float srow[];   // [rows]
     const int n = blockIdx.x;
+    set_mark(mark);
     // Four rows per thread and step (rows is a multiple of 32, the planes 16-byte aligned), two or four loads in flight:
     // a call of few tokens has few workgroups, and one load after another was most of its time (9728 rows x 19 tokens:
     // 17 us; 4096 rows, 4 planes, 65 tokens: the whole call 40.3 -> 26.6 us).
@@ -536,28 +543,65 @@ static int grow(void **p, size_t *have, size_t need, const char *what) {
     return P8X_OK;
 }
 
-struct HipApi {   // p8x_operands.h
-    static bool alloc(void **p, size_t n) { return hipMalloc(p, n) == hipSuccess; }
-    static void release(void *p) { (void)hipFree(p); }
-    static bool synchronize() { return hipDeviceSynchronize() == hipSuccess; }
-    static void clear_error() { (void)hipGetLastError(); }
+// Device calls of p8x_operands.h. A thread may allocate while another captures a graph: these calls are kept out of
+// captures that do not concern them.
+struct AnyCapture {
+    hipStreamCaptureMode m = hipStreamCaptureModeRelaxed;
+    AnyCapture() { (void)hipThreadExchangeStreamCaptureMode(&m); }
+    ~AnyCapture() { (void)hipThreadExchangeStreamCaptureMode(&m); }
 };
+struct HipApi {
+    using Stream = hipStream_t;
+    static bool ok(hipError_t e) {
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e == hipSuccess;
+    }
+    static bool alloc(void **p, size_t n) { AnyCapture r; return hipMalloc(p, n) == hipSuccess; }
+    static void release(void *p) { AnyCapture r; (void)hipFree(p); }
+    static bool synchronize() { AnyCapture r; return hipDeviceSynchronize() == hipSuccess; }
+    static void clear_error() { (void)hipGetLastError(); }
+    static bool host_word(unsigned long long **p) {
+        AnyCapture r;
+        if (!ok(hipHostMalloc((void **)p, sizeof **p, hipHostMallocMapped | hipHostMallocPortable))) return false;
+        **p = 0;
+        return true;
+    }
+    static bool ordered(Stream a, Stream b) { return a == b && a != hipStreamPerThread; }   // that handle names one per thread
+    static bool capturing(Stream st) {
+        hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+        return !ok(hipStreamIsCapturing(st, &s)) || s != hipStreamCaptureStatusNone;
+    }
+};
+
+constexpr int kMaxDevices = 64;
+static OperandBuffer<HipApi> g_operands[kMaxDevices];
+
+bool mm_only_c3(const p8x_tensor *t) {
+    for (int c = 1; c < 8; ++c) if (c != 3 && t->class_tiles[c]) return false;
+    return true;
+}
+// tensors whose operands mm_plan may have decoded first: one row tile's fit (K <= 393216), see there for the classes
+static bool mm_may_decode(const p8x_tensor *t) { return !mm_only_c3(t) && !t->class_tiles[0] && mm_dense_w_bytes(t) <= kMmOperandBytes; }
+void operands_add_user(p8x_tensor *t) {
+    if (!mm_may_decode(t)) return;
+    g_operands[t->device].add_user();
+    t->operand_user = true;
+}
+void operands_drop_user(const p8x_tensor *t) {
+    if (t->operand_user) g_operands[t->device].drop_user();
+}
 
 struct MmPlan {
     int rg;    // 32-token tiles of the row-group GEMM (p8x_mm_rg.hip), which writes y itself; 0: k_mm, below
-    bool dense;   // decode the weights once (k_mm_decode), then k_mm_dense; else k_mm
+    bool dense;   // decode the weights once (k_mm_decode), then k_mm_dense, band by band; else k_mm
     int nti;   // token tiles per wave: the workgroup tile is 256 rows x 32 nti tokens
     int tiles_m, tiles_n, nsplit, kper;
+    int band;  // row tiles of a launch: all of them, or (dense) those whose operands fit kMmOperandBytes
 };
 
 // One workgroup per CU. Estimated time = rounds of workgroups x (the measured prologue + blocks per workgroup x the
 // measured time of one K block of a workgroup tile of the shape) + when planes are used (K split, or rows to
 // un-permute) their traffic (written by k_mm, read by k_mm_finish at ~5 TB/s) and k_mm_finish's launch.
-bool mm_only_c3(const p8x_tensor *t) {
-    for (int c = 1; c < 8; ++c) if (c != 3 && t->class_tiles[c]) return false;
-    return true;
-}
-
 static MmPlan mm_plan(const p8x_tensor *t, int N) {
     const bool c3 = mm_only_c3(t);
     const long slots = num_cus();
@@ -567,21 +611,23 @@ static MmPlan mm_plan(const p8x_tensor *t, int N) {
     const size_t xb = ((size_t)N * t->K * sizeof(_Float16) + 255) & ~(size_t)255;
     const size_t cap = xb < (size_t)P8X_NOALLOC_SCRATCH_BYTES ? (size_t)P8X_NOALLOC_SCRATCH_BYTES - xb : 0;
 #ifdef P8X_TIMELINE
-    MmPlan best{0, false, 4, 0, 0, 1, t->nb};   // the timeline build stamps k_mm's phases: k_mm at every token count
+    MmPlan best{0, false, 4, 0, 0, 1, t->nb, 0};   // the timeline build stamps k_mm's phases: k_mm at every token count
 #else
-    MmPlan best{mm_rg_tiles(t, N), false, 4, 0, 0, 1, t->nb};
+    MmPlan best{mm_rg_tiles(t, N), false, 4, 0, 0, 1, t->nb, 0};
 #endif
     if (best.rg) return best;
     double best_cost = -1.0;
     auto consider = [&](bool dense, int nti, double block_us, double pro_us, double extra_us) {
         const int tiles_m = (t->rows + mm_rows() - 1) / mm_rows(), tiles_n = (N + mm_tok(nti) - 1) / mm_tok(nti);
-        const long base = (long)tiles_m * tiles_n;
+        const int band = dense ? mm_dense_band(t) : tiles_m;
         for (int ns = 1; ns <= std::min(t->nb, 16); ++ns) {
             const int kper = (t->nb + ns - 1) / ns, nsr = (t->nb + kper - 1) / kper;
             if (nsr > 1 && (size_t)nsr * N * t->rows * 4 > cap) continue;
             const bool planes = nsr > 1 || !t->prm_identity;
-            const double cost = (double)((base * nsr + slots - 1) / slots) * (pro_us + kper * block_us) + (planes ? nsr * plane_us + finish_us : 0.0) + extra_us;
-            if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = MmPlan{0, dense, nti, tiles_m, tiles_n, nsr, kper}; }
+            auto rounds = [&](int tiles) { return ((long)tiles * tiles_n * nsr + slots - 1) / slots; };
+            const double cost = (double)(tiles_m / band * rounds(band) + rounds(tiles_m % band)) * (pro_us + kper * block_us) +
+                                (planes ? nsr * plane_us + finish_us : 0.0) + extra_us;
+            if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = MmPlan{0, dense, nti, tiles_m, tiles_n, nsr, kper, band}; }
         }
     };
     // One K block of one workgroup tile and the prologue, us, measured: class 3 at 256 x 256 and 256 x 128; every class
@@ -593,8 +639,9 @@ static MmPlan mm_plan(const p8x_tensor *t, int N) {
     // tiles; the dense kernel alone 1.07 PFLOP/s, the card's library product 1.2). Class 3 keeps k_mm, whose decode is
     // cheaper: 14336 x 4096, 512 tokens 98 (k_mm) and 123 us, 2048 tokens 394 and 399. Class-0 tiles are skipped by k_mm
     // and have no operands: tensors with such tiles keep it.
-    if (!c3 && !t->class_tiles[0])
-        for (int nti = 4; nti <= 6; ++nti) consider(true, nti, nti == 4 ? 3.6 : nti == 5 ? 4.7 : 5.8, 2.0, 5.0 + mm_dense_w_bytes(t) / 4.2e6);
+    if (mm_may_decode(t))
+        for (int nti = 4; nti <= 6; ++nti)
+            consider(true, nti, nti == 4 ? 3.6 : nti == 5 ? 4.7 : 5.8, 2.0, 5.0 + (double)t->nt * kMmTileHalves * sizeof(_Float16) / 4.2e6);
     return best;
 }
 
@@ -620,7 +667,7 @@ int reserve_mul_mat(const p8x_tensor *t, int n_max) {
     int rc;
     if ((rc = grow((void **)&tw->wx16, &tw->wx16_elems, xb, "p8x_mul_mat_reserve: activation workspace"))) return rc;
     if (planes && (rc = grow((void **)&tw->wmm, &tw->wmm_bytes, planes, "p8x_mul_mat_reserve: output planes"))) return rc;
-    if (wb) (void)try_grow<HipApi>(&tw->wbw, &tw->wbw_bytes, wb);   // calls run k_mm without them
+    if (wb) g_operands[t->device].reserve(wb);
     return P8X_OK;
 }
 
@@ -643,10 +690,10 @@ static int finish_lds_attribute() {
 }
 
 // the launches of one prompt GEMM with its workspace given: xr >= N K fp16, wmm >= the plane bytes (unused when the
-// output is written directly), bw the decoded operands' bytes. Without bw a decoded-weights plan runs k_mm with that
-// plan's K split: the same bits.
+// output is written directly), bw the decoded operands' bytes (shared: the lease that bw is of, or null). Without bw a
+// decoded-weights plan runs k_mm with that plan's K split: the same bits.
 static int launch_mul_mat_ws(const p8x_tensor *t, const void *x, int x_dtype, int N, size_t ldx, float *y, size_t ldy, _Float16 *xr,
-                             float *wmm, void *bw, hipStream_t st) {
+                             float *wmm, void *bw, OperandBuffer<HipApi>::Lease *shared, hipStream_t st) {
     MmPlan p = mm_plan(t, N);
     if (p.rg) return launch_mm_rg(t, p.rg, x, x_dtype, N, ldx, y, ldy, xr, st);
     const bool direct = p.nsplit == 1 && t->prm_identity;
@@ -668,24 +715,37 @@ static int launch_mul_mat_ws(const p8x_tensor *t, const void *x, int x_dtype, in
 #ifdef P8X_TIMELINE
     J.tl = timeline_buf();
 #endif
-    J.bw = (const _Float16 *)bw;
+    J.bw = (const _Float16 *)bw; J.g0 = 0;
     const int grid = ((p.tiles_m * p.tiles_n * p.nsplit + kXcds - 1) / kXcds) * kXcds;
     if (p.dense) {
-        if ((rc = launch_mm_decode(t, bw, st)) || (rc = launch_mm_dense(p.nti, J, st))) return rc;
+        constexpr int GPT = mm_rows() / 32;   // row groups of a row tile
+        for (int tm = 0; tm < p.tiles_m; tm += p.band) {
+            J.tiles_m = std::min(p.band, p.tiles_m - tm);
+            J.g0 = tm * GPT;
+            if ((rc = launch_mm_decode(t, J.g0, std::min(J.tiles_m * GPT, t->ng - J.g0), bw, st)) || (rc = launch_mm_dense(p.nti, J, st))) return rc;
+        }
     } else if (!mm_only_c3(t)) hipLaunchKernelGGL((k_mm<kMmCmAll, 4>), dim3(grid), dim3(64 * mm_waves()), 0, st, J);
     else if (p.nti == 8) hipLaunchKernelGGL((k_mm<kMmCmC3, 8>), dim3(grid), dim3(64 * mm_waves()), 0, st, J);
     else hipLaunchKernelGGL((k_mm<kMmCmC3, 4>), dim3(grid), dim3(64 * mm_waves()), 0, st, J);
     if ((rc = hip_check(hipGetLastError(), "k_mm launch"))) return rc;
+    const OperandMark mark = p.dense && shared ? shared->mark() : OperandMark{};
     if (!direct) {
         const size_t lds = 4 * (size_t)t->rows;   // rows < 32768: at most 128 KB
         if ((rc = finish_lds_attribute())) return rc;
         if (x_dtype == P8X_F32)
             hipLaunchKernelGGL(k_mm_finish<float>, dim3(N), dim3(1024), lds, st, (const float *)wmm, p.nsplit, N, t->rows, t->pinv, t->cp, t->cc, t->cv,
-                               (const float *)x, ldx, y, ldy);
+                               (const float *)x, ldx, y, ldy, mark);
         else
             hipLaunchKernelGGL(k_mm_finish<uint16_t>, dim3(N), dim3(1024), lds, st, (const float *)wmm, p.nsplit, N, t->rows, t->pinv, t->cp, t->cc, t->cv,
-                               (const uint16_t *)x, ldx, y, ldy);
-        return hip_check(hipGetLastError(), "k_mm_finish launch");
+                               (const uint16_t *)x, ldx, y, ldy, mark);
+        if ((rc = hip_check(hipGetLastError(), "k_mm_finish launch"))) return rc;
+        if (mark.word) shared->launched();
+        return P8X_OK;
+    }
+    if (mark.word) {
+        hipLaunchKernelGGL(k_mm_mark, dim3(1), dim3(64), 0, st, mark);
+        if ((rc = hip_check(hipGetLastError(), "k_mm_mark launch"))) return rc;
+        shared->launched();
     }
     if (t->ndrows) {
         if (x_dtype == P8X_F32)
@@ -705,8 +765,13 @@ int launch_mul_mat(const p8x_tensor *t, const void *x, int x_dtype, int N, size_
     int rc;
     if ((rc = grow((void **)&tw->wx16, &tw->wx16_elems, xb, "p8x_mul_mat: activation workspace"))) return rc;
     if (pb && (rc = grow((void **)&tw->wmm, &tw->wmm_bytes, pb, "p8x_mul_mat: output planes"))) return rc;
-    return launch_mul_mat_ws(t, x, x_dtype, N, ldx, y, ldy, reinterpret_cast<_Float16 *>(tw->wx16), tw->wmm,
-                             wb && try_grow<HipApi>(&tw->wbw, &tw->wbw_bytes, wb) ? tw->wbw : nullptr, st);
+    OperandBuffer<HipApi>::Lease shared = wb ? g_operands[t->device].take(wb, st) : OperandBuffer<HipApi>::Lease();
+    void *bw = shared.p;
+    // a call that is captured has operands of its own, kept with the tensor as its other workspaces are: the graph may be
+    // replayed beside any other call but those on this tensor
+    if (wb && !bw && HipApi::capturing(st) && try_grow<HipApi>(&tw->wbw, &tw->wbw_bytes, wb)) bw = tw->wbw;
+    return launch_mul_mat_ws(t, x, x_dtype, N, ldx, y, ldy, reinterpret_cast<_Float16 *>(tw->wx16), tw->wmm, bw,
+                             shared.p ? &shared : nullptr, st);
 }
 
 // ------------------------------------------------------------------------------------------------ no-allocation variant
@@ -715,7 +780,6 @@ int launch_mul_mat(const p8x_tensor *t, const void *x, int x_dtype, int N, size_
 // that GPU current, resolved once per device (scratch_resolve) and used everywhere host code passes the array on.
 static __device__ __align__(256) uint8_t scratch[P8X_NOALLOC_SCRATCH_BYTES];
 
-constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
 static void *g_scratch[kMaxDevices];
 
@@ -763,6 +827,6 @@ extern "C" int p8x_mul_mat_noalloc(const p8x_tensor *t, const void *x, int x_dty
     // otherwise, the same bits); every byte read is written earlier in the call
     const size_t w_off = (xb_al + pb + 255) & ~(size_t)255;
     void *bw = wb && w_off + wb <= (size_t)P8X_NOALLOC_SCRATCH_BYTES ? base + w_off : nullptr;
-    return launch_mul_mat_ws(t, x, x_dtype, N, ldx, y, ldy, reinterpret_cast<_Float16 *>(base), reinterpret_cast<float *>(base + xb_al), bw,
+    return launch_mul_mat_ws(t, x, x_dtype, N, ldx, y, ldy, reinterpret_cast<_Float16 *>(base), reinterpret_cast<float *>(base + xb_al), bw, nullptr,
                              (hipStream_t)stream);
 }

@@ -143,6 +143,7 @@ void p8x_release(p8x_tensor *t) {
     for (void *p : {(void *)t->owned, (void *)t->Dl, (void *)t->wy, (void *)t->wglu, (void *)t->wslot, (void *)t->djob, (void *)t->Sg, (void *)t->a2, (void *)t->ic, (void *)t->cp, (void *)t->cc, (void *)t->cv, (void *)t->wq,
                     (void *)t->wd, (void *)t->wsum, (void *)t->wq81, (void *)t->wpart, (void *)t->wcnt, (void *)t->drows, (void *)t->pinv, (void *)t->prmd, (void *)t->wx16, (void *)t->wmm, t->wbw})
         if (p) (void)hipFree(p);
+    operands_drop_user(t);
     delete t;
 }
 
@@ -381,6 +382,7 @@ int p8x_prepare(const void *slot, size_t n, int rows, int K, int on_device, p8x_
     if (bad && (rc = hip_check(hipMemset(t->wcnt, 0, 4), "p8x_prepare: counters"))) return fail(rc);
     if ((rc = upload_job(t))) return fail(rc);
     if ((rc = hip_check(hipDeviceSynchronize(), "p8x_prepare: sync"))) return fail(rc);
+    operands_add_user(t);
     *out = t;
     return P8X_OK;
 }

@@ -61,8 +61,9 @@ struct p8x_tensor {
     size_t wx16_elems = 0;           // capacity in bytes
     float *wmm = nullptr;            // prompt GEMM: K-split partial planes (grown on demand)
     size_t wmm_bytes = 0;
-    void *wbw = nullptr;             // prompt GEMM of many tokens: decoded fp16 operands, 2 rows K bytes (grown on demand)
+    void *wbw = nullptr;             // prompt GEMM of many tokens under graph capture: decoded fp16 operands of a band
     size_t wbw_bytes = 0;
+    bool operand_user = false;       // counted as a user of the GPU's shared operand buffer (p8x_operands.h)
     uint32_t a2_host[512];           // host copy of a2 (batches check that tensors share the tables)
 };
 
@@ -110,6 +111,9 @@ int launch_decode_rotated(const p8x_tensor *t, int dtype, int g0, int gn, int b0
 int launch_dequant(const p8x_tensor *t, int dtype, int row0, int nrows, void *out, size_t ld, hipStream_t st);
 int launch_mul_mat(const p8x_tensor *t, const void *x, int x_dtype, int N, size_t ldx, float *y, size_t ldy, hipStream_t st);
 int reserve_mul_mat(const p8x_tensor *t, int n_max);
+// the tensor as a user of its GPU's operand buffer, at prepare and release
+void operands_add_user(p8x_tensor *t);
+void operands_drop_user(const p8x_tensor *t);
 // the tensor's GemvJob in device memory (t->djob), at prepare
 int upload_job(p8x_tensor *t);
 // device address of the no-allocation scratch array on `device` (hipGetSymbolAddress, once per device)

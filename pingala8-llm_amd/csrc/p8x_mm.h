@@ -78,7 +78,8 @@ struct MmJob {
     const uint32_t *a2;     // [2][256] coset table words (A[f] + h c), h-major, then the same as fp16: entry 2 f + h,
                             // 4 halves
     int N, rows, K, nb, ng;
-    const _Float16 *bw;     // k_mm_dense: the decoded weights (k_mm_decode)
+    const _Float16 *bw;     // k_mm_dense: the decoded weights (k_mm_decode) of the launch's row groups, g0 the first
+    int g0;
     int tiles_m, tiles_n, nsplit, kper, direct;
 #ifdef P8X_TIMELINE
     unsigned long long *tl;
@@ -135,8 +136,11 @@ int mm_rg_tiles(const p8x_tensor *t, int N);                  // 32-token tiles 
 size_t mm_rg_x_bytes(const p8x_tensor *t, int tiles);         // its x' workspace
 // the decoded-weights GEMM (p8x_mm_dense.hip): weight operands decoded once per call, then a dense kernel of
 // 256 rows x 32 nti tokens per workgroup, nti 4 .. 6
-size_t mm_dense_w_bytes(const p8x_tensor *t);
-int launch_mm_decode(const p8x_tensor *t, void *bw, hipStream_t st);
+constexpr int kMmTileHalves = 16 * 64 * 8;             // decoded operands of a weight tile
+constexpr size_t kMmOperandBytes = (size_t)192 << 20;  // at most this much of them at a time: 17408 x 5120 in one band
+int mm_dense_band(const p8x_tensor *t);                // row tiles of a band
+size_t mm_dense_w_bytes(const p8x_tensor *t);          // its operands
+int launch_mm_decode(const p8x_tensor *t, int g0, int gn, void *bw, hipStream_t st);
 int launch_mm_dense(int nti, const MmJob &J, hipStream_t st);
 int launch_mm_rg(const p8x_tensor *t, int tiles, const void *x, int x_dtype, int N, size_t ldx, float *y, size_t ldy, void *xf, hipStream_t st);
 

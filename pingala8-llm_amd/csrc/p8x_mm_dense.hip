@@ -15,11 +15,9 @@
 
 namespace p8x {
 
-// Decoded operands: [row group g][block b][step s][lane][8 halves]: lane (row j = lane & 31, half kh = lane >> 5) of
+// Decoded operands: [row group g of the band][block b][step s][lane][8 halves]: lane (row j = lane & 31, half kh = lane >> 5) of
 // step s holds the eight weights of sorted row 32 g + j at columns 256 b + 128 kh + 8 s .., what v_mfma_f32_32x32x16_f16
-// takes as its second operand. 16 KB per tile; a wave stores and loads a step as 1 KB of consecutive bytes.
-constexpr int kMmTileHalves = 16 * 64 * 8;
-
+// takes as its second operand. 16 KB per tile (kMmTileHalves); a wave stores and loads a step as 1 KB of consecutive bytes.
 constexpr int kMmDecWaves = 8;
 struct MmDecJob {
     const uint32_t *M; const uint16_t *Sg; const uint32_t *D; const uint32_t *a2;
@@ -125,8 +123,8 @@ __global__ __launch_bounds__(64 * mm_waves()) __attribute__((amdgpu_waves_per_eu
     gptr<const half8v> bp[NTJ];
 #pragma unroll
     for (int tj = 0; tj < NTJ; ++tj) {
-        g[tj] = (tm * mm_rows()) / 32 + NTJ * w + tj;   // row groups past the tensor repeat the last (never stored)
-        bp[tj] = as_global(reinterpret_cast<const half8v *>(J.bw + ((size_t)min(g[tj], J.ng - 1) * J.nb + b0) * kMmTileHalves)) + lane;
+        g[tj] = J.g0 + (tm * mm_rows()) / 32 + NTJ * w + tj;   // row groups past the tensor repeat the last (never stored)
+        bp[tj] = as_global(reinterpret_cast<const half8v *>(J.bw + ((size_t)(min(g[tj], J.ng - 1) - J.g0) * J.nb + b0) * kMmTileHalves)) + lane;
     }
     float16v acc[NTI][NTJ];
 #pragma unroll
@@ -208,11 +206,23 @@ __global__ __launch_bounds__(64 * mm_waves()) __attribute__((amdgpu_waves_per_eu
     }
 }
 
-size_t mm_dense_w_bytes(const p8x_tensor *t) { return t->nt * kMmTileHalves * sizeof(_Float16); }
+int mm_dense_band(const p8x_tensor *t) {
+    const int tiles = (t->rows + mm_rows() - 1) / mm_rows();
+    const size_t per = (size_t)(mm_rows() / 32) * t->nb * kMmTileHalves * sizeof(_Float16);
+    const int most = std::max(1, (int)(kMmOperandBytes / per)), bands = (tiles + most - 1) / most;
+    return (tiles + bands - 1) / bands;
+}
 
-int launch_mm_decode(const p8x_tensor *t, void *bw, hipStream_t st) {
-    MmDecJob J{t->M, t->Sg, t->D, t->a2, (_Float16 *)bw, (int)t->nt, (uint32_t)(t->kbytes - offset_D(t->nt)), (uint32_t)(t->nb * t->rows * 2)};
-    const int grid = std::min((int)((t->nt + kMmDecWaves - 1) / kMmDecWaves), 2 * num_cus());
+size_t mm_dense_w_bytes(const p8x_tensor *t) {
+    return (size_t)std::min(mm_dense_band(t) * (mm_rows() / 32), t->ng) * t->nb * kMmTileHalves * sizeof(_Float16);
+}
+
+// operands of row groups g0 .. g0 + gn - 1
+int launch_mm_decode(const p8x_tensor *t, int g0, int gn, void *bw, hipStream_t st) {
+    const size_t t0 = (size_t)g0 * t->nb;
+    const int nt = gn * t->nb;
+    MmDecJob J{t->M + t0, t->Sg + 32 * t0, t->D, t->a2, (_Float16 *)bw, nt, (uint32_t)(t->kbytes - offset_D(t->nt)), (uint32_t)nt * 64u};
+    const int grid = std::min((nt + kMmDecWaves - 1) / kMmDecWaves, 2 * num_cus());
     hipLaunchKernelGGL(k_mm_decode, dim3(grid), dim3(64 * kMmDecWaves), 0, st, J);
     return hip_check(hipGetLastError(), "k_mm_decode launch");
 }

@@ -1,8 +1,10 @@
-// p8x_operands.h -- device memory of the prompt GEMM's decoded fp16 weight operands. A call that gets none runs the
-// kernel that decodes as it multiplies (k_mm): the same bits, slower. Templated on the device calls (HipApi in
-// p8x_gemm.hip), so that the rules can be tested without a GPU.
+// p8x_operands.h -- device memory of the prompt GEMM's decoded fp16 weight operands. They live within one call, so the
+// calls of all tensors on a GPU share one buffer. A call that gets none runs the kernel that decodes as it multiplies
+// (k_mm): the same bits, slower. Templated on the device calls (HipApi in p8x_gemm.hip), so that the rules can be tested
+// without a GPU.
 #pragma once
 #include <cstddef>
+#include <mutex>
 
 namespace p8x {
 
@@ -29,5 +31,100 @@ bool try_grow(void **p, size_t *have, size_t need) {
     *have = need;
     return true;
 }
+
+// What the last kernel of a call that uses the buffer is given: its first workgroup stores n in *word (host memory), which
+// tells that the launches before it have ended.
+struct OperandMark {
+    unsigned long long *word = nullptr, n = 0;
+};
+
+// The buffer that the calls on one GPU share. One call holds it at a time (its lock spans the call's launches), and a word
+// in host memory, which the kernel behind those that read the buffer writes, tells when the GPU is done with it. (An event
+// recorded there took 1.5 to 3 us a call, 33.0 -> 34.5 / 36.0 for 300 tokens of 1024 x 4096; given to the launch as its
+// stop event, it took 30 us of a first call after a pause.) A call on the stream that used it last is ordered behind that
+// use (a stream's work has ended before its handle is another's: hipStreamDestroy waits for it; Api::ordered says which
+// handles name one stream); a call on any other stream gets it only once that use has ended, and nothing otherwise: it
+// neither waits for another stream nor makes its own wait. Calls under stream capture get nothing, since a graph may be
+// replayed beside anything. The memory is given back when the last tensor that can use it is released.
+template <class Api>
+class OperandBuffer {
+public:
+    class Lease {
+    public:
+        explicit Lease(void *p_ = nullptr) : p(p_) {}
+        Lease(Lease &&o) : p(o.p), b(o.b), st(o.st), on(o.on) { o.p = nullptr; o.b = nullptr; }
+        Lease(const Lease &) = delete;
+        Lease &operator=(const Lease &) = delete;
+        ~Lease() { if (b) b->done(st, on); }
+        OperandMark mark() const { return OperandMark{b->word, b->seq}; }
+        void launched() { on = true; }   // the kernel with the mark is on the stream, behind those that use the buffer
+        void *p;   // null: no buffer
+
+    private:
+        friend class OperandBuffer;
+        OperandBuffer *b = nullptr;
+        typename Api::Stream st{};
+        bool on = false;
+    };
+
+    void add_user() {
+        std::lock_guard<std::mutex> lk(mu);
+        ++users;
+    }
+    void drop_user() {
+        std::lock_guard<std::mutex> lk(mu);
+        failed = 0;   // memory came free
+        if (--users || !buf) return;
+        Api::release(buf);   // waits for the device
+        buf = nullptr;
+        bytes = 0;
+        used = false;   // the word stays
+    }
+    // at set-up: the buffer is there for later calls of up to `need` bytes, if the memory is
+    void reserve(size_t need) {
+        std::lock_guard<std::mutex> lk(mu);
+        failed = 0;
+        (void)provide(need);
+    }
+    Lease take(size_t need, typename Api::Stream st) {
+        Lease l;
+        if (Api::capturing(st)) return l;
+        mu.lock();
+        const bool ready = !used || Api::ordered(st, last) || __atomic_load_n(word, __ATOMIC_ACQUIRE) == seq;
+        if (!ready || !provide(need)) {
+            mu.unlock();
+            return l;
+        }
+        ++seq;
+        l.p = buf;
+        l.b = this;
+        l.st = st;
+        return l;
+    }
+
+private:
+    bool provide(size_t need) {
+        if (failed && need >= failed) return false;   // not tried again on every call
+        if (word || Api::host_word(&word)) {
+            if (try_grow<Api>(&buf, &bytes, need)) return true;
+        }
+        failed = need;
+        return false;
+    }
+    void done(typename Api::Stream st, bool on) {
+        last = st;
+        used = on;
+        if (!on) (void)Api::synchronize();   // a launch failed, no mark covers those before it
+        mu.unlock();
+    }
+
+    std::mutex mu;
+    void *buf = nullptr;
+    size_t bytes = 0, failed = 0;
+    unsigned long long *word = nullptr, seq = 0;   // the mark of the last use
+    typename Api::Stream last{};
+    bool used = false;   // launches of the last use may still run
+    int users = 0;
+};
 
 }  // namespace p8x

@@ -6,12 +6,21 @@ import subprocess
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "pingala8-llm_amd", "csrc")
 
 FAKE = r"""
+#include <atomic>
 #include <cassert>
 #include <cstdio>
 #include <cstdlib>
 #include <string>
+#include <thread>
+#include <vector>
 #include "p8x_operands.h"
 struct Fake {   // log: a = alloc, f = free, s = device synchronize, c = error cleared
+    using Stream = int;
+    static bool cap;   // streams are being captured
+    static unsigned long long *word;
+    static bool host_word(unsigned long long **p) { static unsigned long long w; word = *p = &w; return true; }
+    static bool ordered(Stream a, Stream b) { return a == b && a != 0; }
+    static bool capturing(Stream) { return cap; }
     static std::string log;
     static size_t room, held;
     static bool sticky;
@@ -26,7 +35,7 @@ struct Fake {   // log: a = alloc, f = free, s = device synchronize, c = error c
     static bool synchronize() { log += 's'; return true; }
     static void clear_error() { log += 'c'; sticky = false; }
 };
-std::string Fake::log; size_t Fake::room, Fake::held; bool Fake::sticky;
+std::string Fake::log; size_t Fake::room, Fake::held; bool Fake::sticky, Fake::cap; unsigned long long *Fake::word;
 using namespace p8x;
 """
 
@@ -51,4 +60,106 @@ def test_out_of_memory_is_no_error(tmp_path):
     Fake::room = 200; Fake::log.clear();
     assert(try_grow<Fake>(&p, &have, 80) && have == 80 && Fake::held == 80 && Fake::log == "asf");
     Fake::release(p);
+    """)
+
+
+def test_one_buffer_for_all_calls(tmp_path):
+    """calls on one stream reuse the buffer, a call on another stream (or on a handle that may name another) gets it only
+    when the last use has ended, a captured call never; it grows behind a device synchronize and goes back with the last user"""
+    run(tmp_path, r"""
+    OperandBuffer<Fake> b;
+    Fake::room = 300;
+    b.add_user(); b.add_user();
+    OperandMark m;
+    auto call = [&](size_t need, int st) {
+        auto l = b.take(need, st);
+        if (l.p) { m = l.mark(); assert(m.word == Fake::word && m.n > *m.word); l.launched(); }
+        return l.p;
+    };
+    void *p = call(100, 1);
+    assert(p && Fake::log == "a");
+    assert(call(80, 1) == p && !call(80, 2));
+    const OperandMark second = m;
+    *m.word = second.n - 1;            // the first call has ended, the second has not
+    assert(!call(80, 2));
+    *m.word = second.n;
+    assert(call(80, 2) == p && !call(80, 1));
+    assert(Fake::log == "a");
+    assert(call(150, 2) && Fake::held == 150 && Fake::log == "aasf");
+    *m.word = m.n;
+    assert(call(80, 0) && !call(80, 0));   // 0: a handle that names one stream per thread
+    *m.word = m.n;
+    Fake::cap = true;
+    assert(!call(80, 0));
+    Fake::cap = false;
+    assert(call(80, 3));
+    b.drop_user();
+    assert(Fake::held == 150);
+    b.drop_user();
+    assert(Fake::held == 0);
+    Fake::log.clear();
+    b.add_user();
+    assert(call(10, 4) && Fake::log == "a");   // a new buffer knows of no earlier use
+    b.drop_user();
+    """)
+
+
+def test_failed_allocation_is_not_repeated_by_every_call(tmp_path):
+    run(tmp_path, r"""
+    OperandBuffer<Fake> b;
+    Fake::room = 100;
+    b.add_user(); b.add_user();
+    { auto l = b.take(101, 1); assert(!l.p && !Fake::sticky); }
+    Fake::log.clear();
+    { auto l = b.take(200, 1); assert(!l.p); }
+    assert(Fake::log.empty());
+    { auto l = b.take(50, 1); assert(l.p); l.launched(); }        // a smaller one is tried
+    Fake::room = 400;
+    b.reserve(101);                                 // set-up tries again
+    { auto l = b.take(101, 1); assert(l.p); l.launched(); }
+    Fake::room = 400; Fake::log.clear();
+    { auto l = b.take(350, 1); assert(!l.p); }      // beside the 101 held
+    b.drop_user();                                  // a release, too, lets the next call try
+    Fake::room = 500;
+    { auto l = b.take(350, 1); assert(l.p && Fake::held == 350); l.launched(); }
+    b.drop_user();
+    """)
+
+
+def test_use_without_its_mark_waits_for_the_device(tmp_path):
+    """a call whose launches failed before the one that carries the mark"""
+    run(tmp_path, r"""
+    OperandBuffer<Fake> b;
+    Fake::room = 100;
+    b.add_user();
+    { auto l = b.take(10, 1); assert(l.p); }
+    assert(Fake::log == "as");
+    { auto l = b.take(10, 2); assert(l.p); l.launched(); }
+    { auto l = b.take(10, 1); assert(!l.p); }
+    b.drop_user();
+    """)
+
+
+def test_lease_excludes_other_threads(tmp_path):
+    run(tmp_path, r"""
+    OperandBuffer<Fake> b;
+    Fake::room = 100;
+    b.add_user();
+    std::atomic<int> in{0}, most{0};
+    std::vector<std::thread> th;
+    for (int i = 0; i < 4; ++i)
+        th.emplace_back([&] {
+            for (int k = 0; k < 200; ++k) {
+                auto l = b.take(10, 1);
+                if (!l.p) abort();
+                const int n = ++in;
+                if (n > most) most = n;
+                std::this_thread::yield();
+                --in;
+                l.launched();
+            }
+        });
+    for (auto &t : th) t.join();
+    assert(most == 1);
+    b.drop_user();
     """)
