@@ -213,10 +213,19 @@ int p8x_mul_mat_reserve(const p8x_tensor *t, int n_max);
  * loops, harnesses that forbid hipMalloc): p8x_mul_mat with its workspace (fp16 x' and K-split output planes) in a
  * fixed device array of P8X_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends. Allocates nothing and never
  * synchronizes; rejects (P8X_ERR_UNSUPPORTED) a call whose workspace exceeds the array (512 tokens of the Llama-3.1-8B
- * FFN shapes fit). Every call on one GPU shares that GPU's array: calls that overlap on one GPU (other streams, other
- * threads) race; calls ordered on one stream do not. Results equal p8x_mul_mat's. */
+ * FFN shapes fit). Operands that a call decodes first are in buffers (16, 64 and 192 MiB, of the sizes that the prepared
+ * tensors need) allocated at p8x_prepare and given back with the last tensor that can use them; without one the call decodes
+ * as it multiplies. Every call on one GPU shares that GPU's array and buffers: calls that overlap on one GPU (other
+ * streams, other threads) race; calls ordered on one stream do not. Results equal p8x_mul_mat's. */
 #define P8X_NOALLOC_SCRATCH_BYTES (96 << 20)
 int p8x_mul_mat_noalloc(const p8x_tensor *t, const void *x, int x_dtype, int N, size_t ldx, float *y, size_t ldy, void *stream);
+/* The launch plan of a prompt GEMM of N tokens: the kernel of p8x_mul_mat (row groups of up to 64 tokens, weights decoded as
+ * they are multiplied, or decoded first) and of p8x_mul_mat_noalloc (P8X_MM_NONE: rejected), tokens of a workgroup tile, K
+ * ranges, launches of the row bands whose operands fit their buffer, direct = 1 when y is written without output planes,
+ * bytes of a band's operands. */
+enum { P8X_MM_NONE = 0, P8X_MM_ROW_GROUP = 1, P8X_MM_FUSED = 2, P8X_MM_DECODED = 3 };
+typedef struct p8x_mul_mat_info { int kernel, noalloc_kernel, token_tile, nsplit, bands, direct; size_t operand_bytes; } p8x_mul_mat_info;
+int p8x_mul_mat_plan(const p8x_tensor *t, int N, p8x_mul_mat_info *out);
 
 /* ---- grouped GEMV ------------------------------------------------------------------------------------- */
 /* No counterpart in the reference (ggml issues one mul_mat per graph node). A fixed list of independent

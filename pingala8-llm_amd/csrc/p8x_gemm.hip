@@ -574,7 +574,12 @@ struct HipApi {
 };
 
 constexpr int kMaxDevices = 64;
-static OperandBuffer<HipApi> g_operands[kMaxDevices];
+struct DeviceOperands {
+    OperandBuffer<HipApi> shared;   // p8x_mul_mat
+    FixedOperands<HipApi> fixed;    // p8x_mul_mat_noalloc
+};
+static DeviceOperands g_operands[kMaxDevices];
+static_assert(FixedOperands<HipApi>::kSizes[2] == kMmOperandBytes, "a band fits the largest");
 
 bool mm_only_c3(const p8x_tensor *t) {
     for (int c = 1; c < 8; ++c) if (c != 3 && t->class_tiles[c]) return false;
@@ -584,11 +589,14 @@ bool mm_only_c3(const p8x_tensor *t) {
 static bool mm_may_decode(const p8x_tensor *t) { return !mm_only_c3(t) && !t->class_tiles[0] && mm_dense_w_bytes(t) <= kMmOperandBytes; }
 void operands_add_user(p8x_tensor *t) {
     if (!mm_may_decode(t)) return;
-    g_operands[t->device].add_user();
+    g_operands[t->device].shared.add_user();
+    g_operands[t->device].fixed.add_user(mm_dense_w_bytes(t));
     t->operand_user = true;
 }
 void operands_drop_user(const p8x_tensor *t) {
-    if (t->operand_user) g_operands[t->device].drop_user();
+    if (!t->operand_user) return;
+    g_operands[t->device].shared.drop_user();
+    g_operands[t->device].fixed.drop_user();
 }
 
 struct MmPlan {
@@ -667,7 +675,7 @@ int reserve_mul_mat(const p8x_tensor *t, int n_max) {
     int rc;
     if ((rc = grow((void **)&tw->wx16, &tw->wx16_elems, xb, "p8x_mul_mat_reserve: activation workspace"))) return rc;
     if (planes && (rc = grow((void **)&tw->wmm, &tw->wmm_bytes, planes, "p8x_mul_mat_reserve: output planes"))) return rc;
-    if (wb) g_operands[t->device].reserve(wb);
+    if (wb) g_operands[t->device].shared.reserve(wb);
     return P8X_OK;
 }
 
@@ -765,7 +773,7 @@ int launch_mul_mat(const p8x_tensor *t, const void *x, int x_dtype, int N, size_
     int rc;
     if ((rc = grow((void **)&tw->wx16, &tw->wx16_elems, xb, "p8x_mul_mat: activation workspace"))) return rc;
     if (pb && (rc = grow((void **)&tw->wmm, &tw->wmm_bytes, pb, "p8x_mul_mat: output planes"))) return rc;
-    OperandBuffer<HipApi>::Lease shared = wb ? g_operands[t->device].take(wb, st) : OperandBuffer<HipApi>::Lease();
+    OperandBuffer<HipApi>::Lease shared = wb ? g_operands[t->device].shared.take(wb, st) : OperandBuffer<HipApi>::Lease();
     void *bw = shared.p;
     // a call that is captured has operands of its own, kept with the tensor as its other workspaces are: the graph may be
     // replayed beside any other call but those on this tensor
@@ -823,10 +831,26 @@ extern "C" int p8x_mul_mat_noalloc(const p8x_tensor *t, const void *x, int x_dty
         if (rc) return rc;
         base = static_cast<uint8_t *>(scratch_ptr(t->device));
     }
-    // x' first, the output planes after it on a 256-byte boundary, then the decoded weights where they fit (k_mm
-    // otherwise, the same bits); every byte read is written earlier in the call
-    const size_t w_off = (xb_al + pb + 255) & ~(size_t)255;
-    void *bw = wb && w_off + wb <= (size_t)P8X_NOALLOC_SCRATCH_BYTES ? base + w_off : nullptr;
+    // x' first, the output planes after it on a 256-byte boundary; every byte read is written earlier in the call
+    void *bw = wb ? g_operands[t->device].fixed.get(wb) : nullptr;   // null: k_mm, the same bits
     return launch_mul_mat_ws(t, x, x_dtype, N, ldx, y, ldy, reinterpret_cast<_Float16 *>(base), reinterpret_cast<float *>(base + xb_al), bw, nullptr,
                              (hipStream_t)stream);
+}
+
+extern "C" int p8x_mul_mat_plan(const p8x_tensor *t, int N, p8x_mul_mat_info *out) {
+    using namespace p8x;
+    if (!t || !out || N < 1) return set_error(P8X_ERR_ARG, "p8x_mul_mat_plan: null pointer or N %d", N);
+    const MmPlan p = mm_plan(t, N);
+    size_t xb, pb, wb;
+    mm_workspace(t, N, &xb, &pb, &wb);
+    *out = p8x_mul_mat_info{};
+    out->kernel = out->noalloc_kernel = p.rg ? P8X_MM_ROW_GROUP : p.dense ? P8X_MM_DECODED : P8X_MM_FUSED;
+    if (((xb + 255) & ~(size_t)255) + pb > (size_t)P8X_NOALLOC_SCRATCH_BYTES) out->noalloc_kernel = P8X_MM_NONE;
+    else if (p.dense && !g_operands[t->device].fixed.get(wb)) out->noalloc_kernel = P8X_MM_FUSED;
+    out->token_tile = p.rg ? 32 * p.rg : mm_tok(p.nti);
+    out->nsplit = p.nsplit;
+    out->bands = p.rg ? 1 : (p.tiles_m + p.band - 1) / p.band;
+    out->direct = p.rg || (p.nsplit == 1 && t->prm_identity);
+    out->operand_bytes = wb;
+    return P8X_OK;
 }

@@ -1,5 +1,5 @@
 // p8x_operands.h -- device memory of the prompt GEMM's decoded fp16 weight operands. They live within one call, so the
-// calls of all tensors on a GPU share one buffer. A call that gets none runs the kernel that decodes as it multiplies
+// calls of all tensors on a GPU share it. A call that gets none runs the kernel that decodes as it multiplies
 // (k_mm): the same bits, slower. Templated on the device calls (HipApi in p8x_gemm.hip), so that the rules can be tested
 // without a GPU.
 #pragma once
@@ -124,6 +124,48 @@ private:
     unsigned long long *word = nullptr, seq = 0;   // the mark of the last use
     typename Api::Stream last{};
     bool used = false;   // launches of the last use may still run
+    int users = 0;
+};
+
+// The operands of calls that may not allocate: buffers of fixed sizes, allocated when the first tensor that needs one is
+// prepared and given back with the last of all, so a captured call's pointer holds as long as its tensor. Calls that share
+// them are ordered by the caller.
+template <class Api>
+class FixedOperands {
+public:
+    static constexpr size_t kSizes[] = {(size_t)16 << 20, (size_t)64 << 20, (size_t)192 << 20};
+
+    void add_user(size_t need) {
+        std::lock_guard<std::mutex> lk(mu);
+        ++users;
+        for (int i = 0; i < kN; ++i)
+            if (need <= kSizes[i]) {
+                if (!buf[i] && !Api::alloc(&buf[i], kSizes[i])) {
+                    Api::clear_error();
+                    buf[i] = nullptr;
+                }
+                return;
+            }
+    }
+    void drop_user() {
+        std::lock_guard<std::mutex> lk(mu);
+        if (--users) return;
+        for (void *&b : buf) {
+            if (b) Api::release(b);
+            b = nullptr;
+        }
+    }
+    void *get(size_t need) {   // null: none
+        std::lock_guard<std::mutex> lk(mu);
+        for (int i = 0; i < kN; ++i)
+            if (need <= kSizes[i] && buf[i]) return buf[i];
+        return nullptr;
+    }
+
+private:
+    static constexpr int kN = sizeof kSizes / sizeof *kSizes;
+    std::mutex mu;
+    void *buf[kN] = {};
     int users = 0;
 };
 

@@ -16,6 +16,7 @@ LIB_PATH = os.path.join(HERE, "libp8x.so")
 P8X_OK, P8X_ERR_ARG, P8X_ERR_FORMAT, P8X_ERR_HIP, P8X_ERR_UNSUPPORTED, P8X_ERR_NOMEM = range(6)
 F32, F16, BF16, I16 = 0, 1, 2, 3
 ACT_Q8_128, ACT_Q8_1, ACT_X16 = 0, 1, 2
+MM_NONE, MM_ROW_GROUP, MM_FUSED, MM_DECODED = 0, 1, 2, 3   # kernels of a prompt GEMM (mul_mat_plan)
 GEMV_KERNEL_AUTO, GEMV_KERNEL_DOT4, GEMV_KERNEL_MFMA = 0, 1, 2   # p8x_gemv_batch_create_ex
 MAX_COLS = 8
 VR3_TAG = 0x56523300
@@ -26,7 +27,7 @@ EXPORTS = [
     "p8x_vec_dot", "p8x_mul_mat_vec", "p8x_mul_mat_vec_act", "p8x_mul_mat", "p8x_mul_mat_reserve", "p8x_synth_random",
     "p8x_quantize_tensor", "p8x_slot_bytes", "p8x_gemv_batch_create", "p8x_gemv_batch_run", "p8x_gemv_batch_run_stage",
     "p8x_gemv_batch_run_stage_timed",
-    "p8x_gemv_batch_release", "p8x_gemv_batch_info", "p8x_mul_mat_noalloc",
+    "p8x_gemv_batch_release", "p8x_gemv_batch_info", "p8x_mul_mat_noalloc", "p8x_mul_mat_plan",
     "p8x_vr_open", "p8x_vr_count", "p8x_vr_find", "p8x_vr_describe", "p8x_vr_load", "p8x_vr_close", "p8x_vr3_rows",
     "p8x_vr3_expand", "p8x_quantize_x16", "p8x_mul_mat_vec_multi", "p8x_mul_mat_vec_glu", "p8x_mul_mat_vec_multi_act",
     "p8x_mul_mat_vec_glu_act", "p8x_gemv_batch_create_act", "p8x_gemv_batch_create_ex", "p8x_graph_begin", "p8x_decode_tiles",
@@ -61,6 +62,10 @@ class VrDesc(ctypes.Structure):
 class BatchInfo(ctypes.Structure):
     _fields_ = [(f, ctypes.c_int) for f in ("njobs", "ncols", "class_set", "units", "split_jobs", "small_launch", "waves",
                                             "matrix_cores")]
+
+
+class MulMatInfo(ctypes.Structure):
+    _fields_ = [(f, ctypes.c_int) for f in ("kernel", "noalloc_kernel", "token_tile", "nsplit", "bands", "direct")] + [("operand_bytes", ctypes.c_size_t)]
 
 
 class EncodeParams(ctypes.Structure):
@@ -116,6 +121,7 @@ def lib():
     L.p8x_mul_mat.argtypes = [vp, vp, i, i, sz, vp, sz, vp]
     L.p8x_mul_mat_reserve.argtypes = [vp, i]
     L.p8x_mul_mat_noalloc.argtypes = [vp, vp, i, i, sz, vp, sz, vp]
+    L.p8x_mul_mat_plan.argtypes = [vp, i, ctypes.POINTER(MulMatInfo)]
     L.p8x_vr_open.argtypes = [ctypes.POINTER(ctypes.c_char_p), i, ctypes.POINTER(vp)]
     L.p8x_vr_count.argtypes = [vp]
     L.p8x_vr_find.argtypes = [vp, ctypes.c_char_p]
@@ -611,6 +617,12 @@ class Tensor:
     def mul_mat_noalloc_dev(self, x, x_dtype, N, y, ldx=None, ldy=None, stream=None):
         check(lib().p8x_mul_mat_noalloc(self.h, _vp(x), x_dtype, N, ldx or self.K, _vp(y), ldy or self.rows,
                                         stream.h if stream else None), "p8x_mul_mat_noalloc")
+
+    def mul_mat_plan(self, N):
+        """launch plan of a prompt GEMM of N tokens (p8x_mul_mat_info)"""
+        inf = MulMatInfo()
+        check(lib().p8x_mul_mat_plan(self.h, N, ctypes.byref(inf)), "p8x_mul_mat_plan")
+        return {f: getattr(inf, f) for f, _ in MulMatInfo._fields_}
 
     # ---- numpy conveniences (copy in / out, synchronous)
     def dequantize(self, dtype=F32):

@@ -49,6 +49,39 @@ def test_tensors_share_the_operands():
     assert free_bytes() >= base - 4 * MIB
 
 
+@pytest.mark.parametrize("rows,K,N", [(1024, 4096, 300), (4096, 14336, 300), (4096, 14336, 700), (5120, 17408, 900)])
+def test_noalloc_decodes_first_too(rows, K, N):
+    """p8x_mul_mat_noalloc runs p8x_mul_mat's plan on operand buffers of its own, whatever the operands' size, eager and
+    captured (three replays with new inputs), and allocates nothing"""
+    t = tensor(rows + N, rows, K)
+    p = t.mul_mat_plan(N)
+    assert p["kernel"] == p["noalloc_kernel"] == p8x.MM_DECODED
+    rng = np.random.default_rng(N)
+    x = p8x.DeviceBuffer(4 * N * K)
+    ya, yb = p8x.DeviceBuffer(4 * N * rows), p8x.DeviceBuffer(4 * N * rows)
+    t.mul_mat_reserve(N)
+    st = p8x.Stream()
+    g = None
+    for _ in range(3):
+        x.copy_from(p8x.DeviceBuffer.from_numpy(rng.standard_normal((N, K)).astype(np.float32)))
+        ya.fill(0xFF)
+        yb.fill(0xFF)
+        p8x.synchronize()
+        t.mul_mat_dev(x, p8x.F32, N, ya)
+        before = free_bytes()
+        t.mul_mat_noalloc_dev(x, p8x.F32, N, yb)
+        assert free_bytes() == before
+        ref = ya.to_numpy(np.uint32, (N, rows)).copy()
+        assert np.array_equal(yb.to_numpy(np.uint32, (N, rows)), ref)
+        yb.fill(0xFF)
+        p8x.synchronize()
+        g = g or p8x.Graph(lambda s: t.mul_mat_noalloc_dev(x, p8x.F32, N, yb, stream=s), st)
+        g.launch(st)
+        st.sync()
+        assert np.array_equal(yb.to_numpy(np.uint32, (N, rows)), ref)
+    g.release()
+
+
 def test_two_streams_bitwise():
     """three tensors' calls in turn on two streams, without waiting: whoever finds the buffer in use decodes in the GEMM"""
     N = 1500

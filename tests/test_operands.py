@@ -163,3 +163,25 @@ def test_lease_excludes_other_threads(tmp_path):
     assert(most == 1);
     b.drop_user();
     """)
+
+
+def test_fixed_operands(tmp_path):
+    """one buffer per size in use, from the first tensor that needs it to the last of all; out of memory is no error"""
+    run(tmp_path, r"""
+    FixedOperands<Fake> f;
+    const size_t M = 1 << 20;
+    Fake::room = 100 * M;
+    f.add_user(16 * M);
+    void *p = f.get(16 * M);
+    assert(p && Fake::held == 16 * M && !f.get(16 * M + 1));
+    f.add_user(M);
+    assert(f.get(M) == p && Fake::held == 16 * M);
+    f.add_user(16 * M + 1);
+    assert(f.get(64 * M) && f.get(64 * M) != p && Fake::held == 80 * M);
+    f.add_user(100 * M);
+    assert(!f.get(65 * M) && !Fake::sticky);
+    f.drop_user(); f.drop_user(); f.drop_user();
+    assert(f.get(M) == p && Fake::held == 80 * M);   // a captured call may hold either
+    f.drop_user();
+    assert(!f.get(M) && Fake::held == 0);
+    """)
