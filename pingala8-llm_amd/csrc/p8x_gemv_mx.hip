@@ -31,8 +31,8 @@ struct MxJob {
     const int *cp; const uint16_t *cc; const float *cv;
     const void *q; const float *d;    // prepared activations (q8: int8 [ncv][K] + f32 [ncv][nsl]; block_q8_1 [ncv][K / 32]), or null
     const float *ic;
-    const float *x; size_t ldx;       // original activations (quantized here when q is null; clamp delta), may be null with q
-    float *y; size_t ldy;
+    const float *x; unsigned ldx;     // original activations (quantized here when q is null; clamp delta), may be null with q
+    float *y; unsigned ldy;
     float *wpart; unsigned *wcnt; unsigned long long *wslot;
     int rows, K, nb, ng, nsl;
     int ncols, planes;                // output columns; planes 2: x16, column n is multiplied columns 2 n and 2 n + 1
@@ -143,7 +143,7 @@ void k_gemv_mx(MxJob J) {
     BlockLane in{};
     if (!J.q && w < items) {   // the wave's one block to quantize (kMxInline)
         const int n = w / nbk, b = c0 + w % nbk;
-        in.load(J.x + n * J.ldx + 256 * b, J.ic + 256 * b, lane);
+        in.load(J.x + (size_t)n * J.ldx + 256 * b, J.ic + 256 * b, lane);
     }
     CosetTableFill<NT> fill;
     fill.load(J.a2, tid);
@@ -273,10 +273,10 @@ void k_gemv_mx(MxJob J) {
         auto finish = [&](int n, float v) {   // clamp delta on the original activations, original row
             const int ro = as_global(J.prmd)[32 * g + j], r = ro & 0x7FFF;
             if ((ro & 0x8000) && J.x) {
-                const gptr<const float> xr = as_global(J.x) + n * J.ldx;
+                const gptr<const float> xr = as_global(J.x) + (size_t)n * J.ldx;
                 for (int e = as_global(J.cp)[r]; e < as_global(J.cp)[r + 1]; ++e) v += as_global(J.cv)[e] * xr[as_global(J.cc)[e]];
             }
-            as_global_rw(J.y)[n * J.ldy + r] = v;
+            as_global_rw(J.y)[(size_t)n * J.ldy + r] = v;
         };
         if (active && (!counted || wk == 0)) {
             const gptr<float> wpart = as_global_rw(J.wpart);
@@ -371,7 +371,7 @@ int launch_gemv_mx(const p8x_tensor *t, int act, const void *q, const float *d, 
     if (need > t->wpart_floats) return set_error(P8X_ERR_UNSUPPORTED, "gemv: partial workspace too small");
     J.M = t->M; J.Sg = t->Sg; J.D = t->D; J.a2 = t->a2; J.prmd = t->prmd;
     J.cp = t->cp; J.cc = t->cc; J.cv = t->cv;
-    J.q = q; J.d = d; J.ic = t->ic; J.x = x; J.ldx = ldx; J.y = y; J.ldy = ldy;
+    J.q = q; J.d = d; J.ic = t->ic; J.x = x; J.ldx = (unsigned)ldx; J.y = y; J.ldy = (unsigned)ldy;
     J.wpart = t->wpart; J.wcnt = t->wcnt; J.wslot = t->wslot;
     J.rows = t->rows; J.K = t->K; J.nb = t->nb; J.ng = t->ng; J.nsl = t->nsl; J.ncols = ncols; J.planes = planes;
     J.dbytes = (uint32_t)(t->kbytes - offset_D(t->nt));

@@ -478,6 +478,13 @@ int p8x_mul_mat_vec_act(const p8x_tensor *t, int act, const float *x, int ncols,
         return set_error(P8X_ERR_ARG, "p8x_mul_mat_vec: ldx %zu ldy %zu (x 16-byte aligned, ldx %% 4 == 0)", ldx, ldy);
     hipStream_t st = (hipStream_t)stream;
     int rc;
+    if (act == P8X_ACT_X16 && 2 * ncols > P8X_MAX_COLS)
+        return set_error(P8X_ERR_ARG, "p8x_mul_mat_vec: x16 takes at most %d columns", P8X_MAX_COLS / 2);
+    if (ncols > 1 && (ldx >> 32 || ldy >> 32)) {   // the kernels hold column strides in 32 bits: one column a call
+        for (int n = 0; n < ncols; ++n)
+            if ((rc = p8x_mul_mat_vec_act(t, act, x + n * ldx, 1, ldx, y + n * ldy, ldy, stream))) return rc;
+        return P8X_OK;
+    }
     if (act == P8X_ACT_Q8_128)   // one launch: every task quantizes its chunk of x itself (same arithmetic as the prep)
         return launch_gemv(t, act, nullptr, nullptr, ncols, x, ldx, y, ldy, nullptr, st);
     // Within a graph evaluation (p8x_graph_begin) x16 and block_q8_1 prepare x in a launch of their own, and a later
@@ -490,7 +497,6 @@ int p8x_mul_mat_vec_act(const p8x_tensor *t, int act, const float *x, int ncols,
         return launch_gemv_mx(t, act, blk, nullptr, ncols, 1, x, ldx, y, ldy, st);
     }
     if (act == P8X_ACT_X16) {
-        if (2 * ncols > P8X_MAX_COLS) return set_error(P8X_ERR_ARG, "p8x_mul_mat_vec: x16 takes at most %d columns", P8X_MAX_COLS / 2);
         const size_t qb = ((size_t)2 * ncols * t->K + 255) & ~(size_t)255;
         uint8_t *c = act_reuse(t, act, x, ncols, ldx, qb + (size_t)8 * ncols * t->nsl, st, &have);
         int8_t *q = reinterpret_cast<int8_t *>(c);

@@ -66,14 +66,13 @@ def test_gemv_mx_padded_strides():
     assert np.array_equal(Y[:, :rows], t.mul_mat_vec(np.ascontiguousarray(X[:, :K])))
 
 
-@pytest.mark.parametrize("act,n", [("x16", 2), ("q81", 2), ("q8", 3)])
+@pytest.mark.parametrize("act,n", [("x16", 2), ("q81", 2), ("q8", 2)])
 def test_gemv_mx_strides_past_32_bits(act, n):
-    """columns 2^32 + 64 (three columns: 2^31 + 64) elements apart"""
-    rows, K, ld = 288, 1024, 1 << 32 if n == 2 else 1 << 31
-    ld += 64   # a stride cut to 32 bits would land inside the buffers
+    """columns 2^32 + 64 elements apart (a stride cut to 32 bits lands inside the buffers): each column's own call"""
+    rows, K, ld = 288, 1024, (1 << 32) + 64
     t = p8x.Tensor(p8x.synth_random(1, rows, K, class_p=MIX, nd=6), rows, K)
     X = np.random.default_rng(n).standard_normal((n, K)).astype(np.float32)
-    ref = t.mul_mat_vec(X, act=ACT[act][0])
+    ref = np.concatenate([t.mul_mat_vec(c, act=ACT[act][0]).reshape(1, rows) for c in X])
     x, y = p8x.DeviceBuffer(4 * ((n - 1) * ld + K)), p8x.DeviceBuffer(4 * ((n - 1) * ld + rows))
 
     def copy(dst, src, nbytes, kind):
