@@ -898,21 +898,16 @@ static bool only_class3(const p8x_tensor *t) {
 }
 
 constexpr int kLo46 = (1 << 4) | (1 << 6);
-// every tile of class 0-3, or also 4 and 6 with a codebook and scales that keep the integer stages exact: the
-// integer-butterfly dequantizer; *cm = its class set
-static bool lo_classes(const p8x_tensor *t, int *cm) {
+// the integer-butterfly dequantizer for nt tiles of a tensor: class 0-3, or also 4 and 6 with a codebook that keeps the
+// integer stages exact; *cm = its class set
+static bool lo_classes(const p8x_tensor *t, size_t nt, int *cm) {
     *cm = 0;
     for (int c = 1; c < 8; ++c) if (t->class_tiles[c]) *cm |= 1 << c;
     if ((*cm & ((1 << 5) | (1 << 7))) || !t->scales_plain) return false;
-    if (!(*cm & kLo46)) return true;
-    // a wave takes a tile in about 8 us however few there are, k_dequant a little less (256 x 512: 13.2 and 12.7 us)
-    if (t->nt < (size_t)num_cus()) return false;
-    for (int i = 0; i < 512; ++i)
-        for (int e = 0; e < 4; ++e) {
-            const int v = (int8_t)(t->a2_host[i] >> (8 * e));
-            if (v > kLo46Max || v < -kLo46Max) return false;
-        }
-    return true;
+    // Fewer tiles than CUs keep k_dequant: a wave here takes 5 us more for a tile whose rows carry clamp deltas (one row
+    // group of 4096 x 14336, two rows out: 14.6 us with such a row, 9.3 without, k_dequant 11.4 and 11.1; 512 x 512: 11.9
+    // and 12.9).
+    return !(*cm & kLo46) || (nt >= (size_t)num_cus() && t->book_max <= kLo46Max);
 }
 
 template <int CM>
@@ -963,7 +958,7 @@ int launch_dequant(const p8x_tensor *t, int dtype, int row0, int nrows, void *ou
         a.g0 = lo; a.gn = hi - lo + 1; a.nt = (size_t)a.gn * a.bn;
     }
     int cm;
-    if (dtype != P8X_F32 && lo_classes(t, &cm)) {
+    if (dtype != P8X_F32 && lo_classes(t, a.nt, &cm)) {
         constexpr int kLo = (1 << 1) | (1 << 2) | (1 << 3);
         const int grid = (int)std::min<size_t>((a.nt + kLoWaves - 1) / kLoWaves, (size_t)num_cus() * (cm & kLo46 ? kLo46Per : 4));
         if (only_class3(t)) launch_deq_lo<(1 << 3)>(dtype, a, grid, st);

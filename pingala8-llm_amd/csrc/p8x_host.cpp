@@ -265,6 +265,8 @@ int p8x_prepare(const void *slot, size_t n, int rows, int K, int on_device, p8x_
                 if ((size_t)(M[i] & 0x1FFFFFFFu) != i * t->lin_words) t->lin_words = 0;
         }
     memcpy(t->a2_host, a2.data(), sizeof t->a2_host);
+    for (const uint32_t w : t->a2_host)
+        for (int e = 0; e < 4; ++e) t->book_max = std::max(t->book_max, std::abs((int)(int8_t)(w >> (8 * e))));
     (void)hipGetDevice(&t->device);
     if ((rc = scratch_resolve(t->device))) { delete t; return rc; }   // set-up of the no-allocation entry point
     if ((rc = act_cache_resolve(t->device))) { delete t; return rc; }   // and of the prepared-activation reuse

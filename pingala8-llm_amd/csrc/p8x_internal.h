@@ -33,6 +33,7 @@ struct p8x_tensor {
     uint16_t *prmd = nullptr;        // sorted row -> original row, bit 15 set when that row carries clamp-delta entries
     bool prm_identity = false;
     bool scales_plain = true;        // every row scale is finite with a clear sign (checked at prepare)
+    int book_max = 0;                // largest |A[f] + h c| of the codebook and its coset
     // device metadata built at prepare
     uint32_t *a2 = nullptr;          // [2][256]: A[f] + h c (bytewise), h-major; then the same as fp16 [256][2][4]
     float *ic = nullptr;             // sg / c per column [K]
