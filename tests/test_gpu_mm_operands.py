@@ -105,6 +105,32 @@ def test_two_streams_bitwise():
         assert np.array_equal(y.to_numpy(np.uint32, (N, 4096)), r)
 
 
+@pytest.mark.parametrize("rows,K,N,permute", [(4096, 4096, 1345, True), (8192, 1024, 641, False)])
+def test_busy_buffer_runs_k_mm(rows, K, N, permute):
+    """a call that finds the buffer in use on another stream (milliseconds of calls are queued there) decodes in the GEMM, on
+    the K ranges of the decoded plan: the same bits; afterwards the buffer is free for this stream too"""
+    t = p8x.Tensor(p8x.synth_random(N, rows, K, class_p=MIX, nd=5, permute=permute), rows, K)
+    a = tensor(1)
+    assert t.mul_mat_plan(N)["kernel"] == p8x.MM_DECODED
+    x, xa = (p8x.DeviceBuffer.from_numpy(np.random.default_rng(i).standard_normal(s).astype(np.float32)) for i, s in enumerate(((N, K), (1500, 4096))))
+    y, ya = p8x.DeviceBuffer(4 * N * rows), p8x.DeviceBuffer(4 * 1500 * 4096)
+    t.mul_mat_reserve(N)
+    a.mul_mat_reserve(1500)
+    t.mul_mat_dev(x, p8x.F32, N, y)
+    p8x.synchronize()
+    ref = y.to_numpy(np.uint32, (N, rows)).copy()
+    s1, s2 = p8x.Stream(), p8x.Stream()
+    for busy in (True, False):
+        y.fill(0xFF)
+        p8x.synchronize()
+        if busy:
+            for _ in range(60):
+                a.mul_mat_dev(xa, p8x.F32, 1500, ya, stream=s1)
+        t.mul_mat_dev(x, p8x.F32, N, y, stream=s2)
+        p8x.synchronize()
+        assert np.array_equal(y.to_numpy(np.uint32, (N, rows)), ref)
+
+
 def test_captured_beside_eager():
     """a captured call replayed on one stream while another tensor's eager calls use the shared buffer on a second one"""
     N, rows, K = 640, 2048, 4096
