@@ -572,6 +572,11 @@ __device__ __forceinline__ void gemv_rows_out(const GemvJob &J, int g, int ks, i
     }
 }
 
+// the instantiation that a call with x alone takes (launch_gemv); the others are given quantized activations
+__host__ __device__ constexpr bool gemv_quantizes(int ncol, int act, bool partials, int cm) {
+    return ncol == 2 && act == P8X_ACT_Q8_128 && !partials && cm == kCmAll;
+}
+
 template <int NCOL, int ACT, bool PARTIALS, int CM>
 __global__ __launch_bounds__(64 * gemv_waves(NCOL, ACT, PARTIALS, CM))
 __attribute__((amdgpu_waves_per_eu(gemv_waves_per_eu(NCOL, ACT, PARTIALS, CM), gemv_waves_per_eu(NCOL, ACT, PARTIALS, CM))))
@@ -579,6 +584,7 @@ void k_gemv(GemvJob job0, int total_tasks, const uint32_t *__restrict__ a2) {
     __shared__ GemvSmem<NCOL, ACT> sm;   // static: the table sits at LDS address 0 at compile time
     constexpr int WAVES = gemv_waves(NCOL, ACT, PARTIALS, CM), NT = 64 * WAVES;
     constexpr int NSC = GemvSmem<NCOL, ACT>::kScales / NCOL;
+    constexpr bool QUANT = gemv_quantizes(NCOL, ACT, PARTIALS, CM);
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     TaskCtx<NCOL, ACT> c;
     c.hs = lane >> 5; c.j = lane & 31;
@@ -597,13 +603,13 @@ void k_gemv(GemvJob job0, int total_tasks, const uint32_t *__restrict__ a2) {
         bool scales_staged = false;
         if constexpr (gemv_quad_loads<ACT, PARTIALS>()) {
             // [n][block][half][64]: word i of a half = activation word (i & 31) of that half
-            if (J.q) {
+            if (!QUANT || J.q) {
                 for (int i = tid; i < NCOL * c.nbl * 128; i += NT) {
                     const int n = i / (c.nbl * 128), wi = i % (c.nbl * 128);
                     const int src = (wi >> 7) * 64 + ((wi >> 6) & 1) * 32 + (wi & 31);
                     sm.xq[n * (kXBytes / 4 / NCOL) + wi] = as_global(reinterpret_cast<const uint32_t *>((const int8_t *)J.q + (size_t)n * J.K + 256 * c.b0))[src];
                 }
-            } else {   // the chunk's blocks quantized here, one wave per (column, block): no separate prep launch
+            } else if constexpr (QUANT) {   // the chunk's blocks quantized here, one wave per (column, block): no separate prep launch
                 for (int pi = w; pi < NCOL * c.nbl; pi += WAVES) {
                     const int n = pi / c.nbl, bl = pi % c.nbl;
                     uint32_t packed;
@@ -689,10 +695,9 @@ static int launch_gemv_t(const GemvJob &job0, int tasks, const uint32_t *a2, hip
 // fixed-order fix-up of the multi-column kernel (agent-coherent partial rows, an arrival counter, the last
 // arrival sums the chunks in order).
 constexpr int kRgMaxBlocks = 112;   // activation blocks in LDS (columns x blocks of the K-chunk)
-// up to two columns: 16 waves at 128 VGPRs; more (instantiable; such calls run on the matrix cores): 8 at 256
-__host__ __device__ constexpr int rg_waves(int ncol) { return ncol <= 2 ? 16 : 8; }
+constexpr int kRgWaves = 16;   // at 128 VGPRs, one or two columns
 
-template <int NCOL, int WAVES = rg_waves(NCOL)>
+template <int NCOL, int WAVES = kRgWaves>
 struct RgSmem {
     static constexpr int kXW = kRgMaxBlocks * 128 / NCOL, kNSC = 2 * kRgMaxBlocks / NCOL;   // per-column strides
     uint32_t tab[kTabWords];             // LDS address 0
@@ -703,7 +708,7 @@ struct RgSmem {
 
 // quantize the wave's items w, w + 16, ... (item i = column i / nbk, block i % nbk of the chunk; loaded in `in`)
 // into the LDS activation layout, G items at a time
-template <int G, int NCOL, int WAVES = rg_waves(NCOL), int RQ = kRgMaxBlocks / WAVES>
+template <int G, int NCOL, int WAVES = kRgWaves, int RQ = kRgMaxBlocks / WAVES>
 __device__ __forceinline__ void rg_quantize(int nbk, RgSmem<NCOL> &sm, const BlockLane (&in)[RQ], int w, int lane) {
 #pragma unroll
     for (int i0 = 0; i0 < RQ; i0 += G) {
@@ -784,7 +789,7 @@ __device__ __forceinline__ void glu_meet(const RgJobs &R, int jb, int r, float v
 // team t takes row group g0 + t * (workgroups per chunk) over the chunk, so that a workgroup with several row
 // groups streams them together instead of one after another. The activations, K plan and rotation come from job 0.
 template <int CM, bool SPLIT, int NCOL, bool TEAMS, bool MULTI>
-__global__ __launch_bounds__(64 * rg_waves(NCOL)) __attribute__((amdgpu_waves_per_eu(rg_waves(NCOL) / 4, rg_waves(NCOL) / 4)))
+__global__ __launch_bounds__(64 * kRgWaves) __attribute__((amdgpu_waves_per_eu(kRgWaves / 4, kRgWaves / 4)))
 void k_gemv_rg(RgJobs jobs, const uint32_t *__restrict__ a2, int gc_) {
 #ifdef P8X_TIMELINE
     unsigned long long stamp[7] = {0, 0, 0, 0, 0, 0, 0};
@@ -792,7 +797,7 @@ void k_gemv_rg(RgJobs jobs, const uint32_t *__restrict__ a2, int gc_) {
     __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #endif
     const int gc = TEAMS ? gc_ : 1;   // without teams: one row group at a time, all waves on it
-    constexpr int WAVES = rg_waves(NCOL), RQ = kRgMaxBlocks / WAVES;
+    constexpr int WAVES = kRgWaves, RQ = kRgMaxBlocks / WAVES;
     __shared__ RgSmem<NCOL> sm;
     // the argument fields the x loads need, requested in the first round of scalar loads with the job ranges
     // (left to the scheduler, some land in a second round behind the job selection's branches)
@@ -992,9 +997,9 @@ static int launch_gemv_rg_t(const RgJobs &jobs_, int ng, const uint32_t *a2, hip
     const int nks = jobs.j0.nks;
     // several jobs: each takes ceil(its row groups / per) workgroups per K-chunk (wgbase, set by the caller)
     const int grid = MULTI ? jobs.wgbase[4] : (ng + per - 1) / per * nks;
-    if (nks > 1) hipLaunchKernelGGL((k_gemv_rg<CM, true, NCOL, false, MULTI>), dim3(grid), dim3(64 * rg_waves(NCOL)), 0, st, jobs, a2, 1);
-    else if (gc > 1) hipLaunchKernelGGL((k_gemv_rg<CM, false, NCOL, true, MULTI>), dim3(grid), dim3(64 * rg_waves(NCOL)), 0, st, jobs, a2, gc);
-    else hipLaunchKernelGGL((k_gemv_rg<CM, false, NCOL, false, MULTI>), dim3(grid), dim3(64 * rg_waves(NCOL)), 0, st, jobs, a2, 1);
+    if (nks > 1) hipLaunchKernelGGL((k_gemv_rg<CM, true, NCOL, false, MULTI>), dim3(grid), dim3(64 * kRgWaves), 0, st, jobs, a2, 1);
+    else if (gc > 1) hipLaunchKernelGGL((k_gemv_rg<CM, false, NCOL, true, MULTI>), dim3(grid), dim3(64 * kRgWaves), 0, st, jobs, a2, gc);
+    else hipLaunchKernelGGL((k_gemv_rg<CM, false, NCOL, false, MULTI>), dim3(grid), dim3(64 * kRgWaves), 0, st, jobs, a2, 1);
     return hip_check(hipGetLastError(), "k_gemv_rg launch");
 }
 

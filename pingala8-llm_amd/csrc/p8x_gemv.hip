@@ -53,29 +53,14 @@ __global__ __launch_bounds__(64) void k_act_x16(const float *__restrict__ x, siz
     const int b = blockIdx.x, n = blockIdx.y, lane = threadIdx.x;
     BlockLane in;
     in.load(x + (size_t)n * ldx + 256 * b, ic + 256 * b, lane);
-    float v[4];
-    rotate_block_lane(in, lane, v);
-    float am = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-    am = half_wave_max(am, lane);
-    const float dd = div_rn(am, 8191.f);
-    const float id = dd > 0.f ? div_rn(1.f, dd) : 0.f;
-    int hi[4], lo[4], s_hi = 0, s_lo = 0;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int q = __float2int_rn(v[e] * id);
-        hi[e] = (q + 64) >> 7;
-        lo[e] = q - 128 * hi[e];
-        s_hi += hi[e];
-        s_lo += lo[e];
-    }
-    auto pack = [](const int (&a)[4]) {
-        return (uint32_t)(uint8_t)a[0] | ((uint32_t)(uint8_t)a[1] << 8) | ((uint32_t)(uint8_t)a[2] << 16) | ((uint32_t)(uint8_t)a[3] << 24);
-    };
+    uint32_t ph, pl;
+    float dd;
+    quantize_loaded_x16(in, lane, ph, pl, dd);
     const size_t qo = (size_t)n * qstride + 256 * b;
-    reinterpret_cast<uint32_t *>(qh + qo)[lane] = pack(hi);
-    reinterpret_cast<uint32_t *>(ql + qo)[lane] = pack(lo);
-    s_hi = half_wave_sum(s_hi, lane);
-    s_lo = half_wave_sum(s_lo, lane);
+    reinterpret_cast<uint32_t *>(qh + qo)[lane] = ph;
+    reinterpret_cast<uint32_t *>(ql + qo)[lane] = pl;
+    const int s_hi = half_wave_sum(__builtin_amdgcn_sdot4((int)ph, 0x01010101, 0, false), lane);
+    const int s_lo = half_wave_sum(__builtin_amdgcn_sdot4((int)pl, 0x01010101, 0, false), lane);
     const int nsl = K / 128;
     if ((lane & 31) == 0) {
         const size_t so = (size_t)n * (qstride / 128) + 2 * b + (lane >> 5);
@@ -233,13 +218,13 @@ int launch_gemv(const p8x_tensor *t, int act, const void *q, const float *d, int
         // one linear, x quantized in the launch
         int kc;
         const int nks = rg_plan(t, ncols, &kc);
-        if (nks == 1 || (size_t)nks * ncols * t->rows <= t->wpart_floats) {
-            RgJobs R{};
-            fill_job(R.j0, t, nullptr, nullptr, x, ldx, y, ldy, nullptr, nks, kc, 1, 0);
-            R.njobs = 1;
-            return launch_gemv_rg(ncols, cm, R, t->ng, t->a2, st);
-        }
+        if (nks > 1 && (size_t)nks * ncols * t->rows > t->wpart_floats) return set_error(P8X_ERR_UNSUPPORTED, "gemv: partial workspace too small");
+        RgJobs R{};
+        fill_job(R.j0, t, nullptr, nullptr, x, ldx, y, ldy, nullptr, nks, kc, 1, 0);
+        R.njobs = 1;
+        return launch_gemv_rg(ncols, cm, R, t->ng, t->a2, st);
     }
+    if (!q && !gemv_quantizes(ncols, act, false, cm)) return set_error(P8X_ERR_ARG, "gemv: %d columns without activations", ncols);
     const GemvPlan p = gemv_plan(t, ncols, act, false);
     if (p.nks > 1 && (size_t)p.nks * ncols * t->rows > t->wpart_floats) return set_error(P8X_ERR_UNSUPPORTED, "gemv: partial workspace too small");
     GemvJob job0;

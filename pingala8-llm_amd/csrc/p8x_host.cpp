@@ -317,7 +317,7 @@ int p8x_prepare(const void *slot, size_t n, int rows, int K, int on_device, p8x_
             const GemvPlan plan = gemv_plan(t, nc, act, false);
             if (plan.nks > 1) t->wpart_floats = std::max(t->wpart_floats, (size_t)plan.nks * nc * rows);
             int kc;
-            const int rn = rg_plan(t, nc, &kc);
+            const int rn = nc <= 2 ? rg_plan(t, nc, &kc) : 1;   // more columns take other kernels
             if (rn > 1) t->wpart_floats = std::max(t->wpart_floats, (size_t)rn * nc * rows);
             for (int planes = 1; planes * nc <= P8X_MAX_COLS && planes <= 2; ++planes)
                 t->wpart_floats = std::max(t->wpart_floats, mx_part_floats(t, nc, planes));

@@ -86,7 +86,7 @@ __device__ __forceinline__ void step_stage(kptr<const StepStage> sp, int v, RgSm
                                            , u64 *rec
 #endif
 ) {
-    constexpr int WAVES = rg_waves(1), RQ = kRgMaxBlocks / WAVES;
+    constexpr int WAVES = kRgWaves, RQ = kRgMaxBlocks / WAVES;
     // this workgroup's job, its index among the job's workgroups and their count
     const int jb = (v >= sp->R.wgbase[1]) + (v >= sp->R.wgbase[2]) + (v >= sp->R.wgbase[3]);
     const int wb = pick(jb, sp->R.wgbase[0], sp->R.wgbase[1], sp->R.wgbase[2], sp->R.wgbase[3]);
@@ -304,7 +304,7 @@ __device__ __forceinline__ bool step_barrier(unsigned *words, unsigned spin, uns
 }
 
 template <int CM>
-__global__ __launch_bounds__(64 * rg_waves(1)) __attribute__((amdgpu_waves_per_eu(rg_waves(1) / 4, rg_waves(1) / 4)))
+__global__ __launch_bounds__(64 * kRgWaves) __attribute__((amdgpu_waves_per_eu(kRgWaves / 4, kRgWaves / 4)))
 void k_step(const StepStage *__restrict__ stages, int nst, unsigned *words, unsigned spin, const uint32_t *__restrict__ a2
 #ifdef P8X_TIMELINE
             , u64 *tl
@@ -317,7 +317,7 @@ void k_step(const StepStage *__restrict__ stages, int nst, unsigned *words, unsi
     if (tid == 0) run_s = ld_agent(words + kSwRuns) + 1u;
     // the table once for the whole chain (each stage's barrier after its quantization orders these writes
     // before the first lookup)
-    build_coset_table<64 * rg_waves(1)>(sm.tab, a2, tid);
+    build_coset_table<64 * kRgWaves>(sm.tab, a2, tid);
     __syncthreads();
     const unsigned run = run_s, per_run = (unsigned)(nst - 1);
     bool ok = true;
@@ -364,7 +364,7 @@ static int launch_step_t(const StepStage *stages, int nst, unsigned *words, unsi
 #else
     void *args[] = {(void *)&stages, (void *)&nst, (void *)&words, (void *)&spin, (void *)&a2};
 #endif
-    return hip_check(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(&k_step<CM>), dim3(grid), dim3(64 * rg_waves(1)), args,
+    return hip_check(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(&k_step<CM>), dim3(grid), dim3(64 * kRgWaves), args,
                                                 0, st),
                      "k_step cooperative launch");
 }
@@ -441,8 +441,8 @@ int p8x_step_create(const p8x_step_stage *stages, int n, p8x_step **out) {
     for (int s = 0; s < n; ++s) {
         for (int i = 0; i < stages[s].n; ++i) sp->keep.push_back(stages[s].tensors[i]);
     }
-    int rc = sp->cm == kCmC3 ? occupancy_grid(&k_step<kCmC3>, 64 * rg_waves(1), &sp->grid, "k_step occupancy")
-                             : occupancy_grid(&k_step<kCmAll>, 64 * rg_waves(1), &sp->grid, "k_step occupancy");
+    int rc = sp->cm == kCmC3 ? occupancy_grid(&k_step<kCmC3>, 64 * kRgWaves, &sp->grid, "k_step occupancy")
+                             : occupancy_grid(&k_step<kCmAll>, 64 * kRgWaves, &sp->grid, "k_step occupancy");
     if (!rc && hipMalloc((void **)&sp->dstages, sizeof(StepStage) * n) != hipSuccess) rc = set_error(P8X_ERR_NOMEM, "p8x_step_create: hipMalloc stages");
     if (!rc) rc = hip_check(hipMemcpy(sp->dstages, hs.data(), sizeof(StepStage) * n, hipMemcpyHostToDevice), "p8x_step_create: stages");
     if (!rc && hipMalloc((void **)&sp->words, kSyncWords * sizeof(unsigned)) != hipSuccess) rc = set_error(P8X_ERR_NOMEM, "p8x_step_create: hipMalloc sync");
