@@ -129,9 +129,9 @@ int p8x_vec_dot_rows(const p8x_tensor *t, int act, const void *q, const float *d
 /* y = W x for 1..8 columns (vr_mul_mat_vec, CPU.patch:4466-4521): activation prep + fused decode-GEMV +
  * un-permute + clamp delta. x [ncols][ldx] f32, y [ncols][ldy] f32, original rows. One launch for one column; several
  * columns on the matrix cores, with the activations quantized in that launch or (more than a block per wave) by one
- * before it. Deterministic. The K-chunk partial rows, arrival counters and meeting slots live
- * in the tensor's handle: calls on one tensor from different streams must not overlap (on one stream they are
- * ordered); counters and slots are put back by each call. Records kernel launches only (capture-safe). */
+ * before it. Deterministic. The activations that a launch of their own quantizes, the K-chunk partial
+ * rows, arrival counters and meeting slots live in the tensor's handle: calls on one tensor from different streams must not
+ * overlap (on one stream they are ordered); counters and slots are put back by each call. Records kernel launches only (capture-safe). */
 int p8x_mul_mat_vec(const p8x_tensor *t, const float *x, int ncols, size_t ldx, float *y, size_t ldy, void *stream);
 /* the same with the activation mode chosen: P8X_ACT_Q8_128 (as p8x_mul_mat_vec), P8X_ACT_Q8_1 (ggml block_q8_1 of x')
  * or P8X_ACT_X16 (1..4 columns: both planes of each column as two columns of one GEMV, summed, then the clamp delta; the

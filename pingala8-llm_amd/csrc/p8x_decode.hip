@@ -607,10 +607,11 @@ __global__ __launch_bounds__(kLoThreads) __attribute__((amdgpu_waves_per_eu(4, 4
 //   * up to stage 8 (sums of 16 values: 16 * 510 * 2047 < 2^24) the reference's sums are exact and equal the integers
 //     times S; stage 16 is the integer butterfly and the one multiply by S (it adds two exact values: RN((I_a +- I_b) S));
 //   * stages 32, 64 and 128 are the reference's f32 additions on the reference's operands.
-// A tensor with such a scale, a wider codebook or classes 5 or 7 goes through k_dequant. 4096 x 14336 to
-// fp16: the ffn_down mix (classes 2, 3 and 4) 60.7 -> 44.7 us a call, class 6 66.1 -> 52.0 against k_dequant (classes 0-3:
-// 33.4 in k_dequant_lo); 1024 x 4096 13.8 -> 13.0. Bound by the decode's VALU and the staging waits, as k_dequant_lo; it
-// needs 168 registers, three workgroups per CU.
+// A tensor with such a scale, a wider codebook or classes 5 or 7 goes through k_dequant. 4096 x 14336 to fp16, the kernel
+// alone: the ffn_down mix (classes 2, 3 and 4) 60.7 -> 44.7 us, class 6 66.1 -> 52.0 against k_dequant (classes 0-3: 33.4 in
+// k_dequant_lo); 1024 x 4096 13.8 -> 13.0. Bound by the decode's VALU and its waits: at 168 registers (three workgroups
+// per CU) 16 are spilled (18 with class 6) and reloaded between a tile's decode and its outputs, and a tile starts with a
+// wait for every memory operation in flight.
 constexpr int kLo46Max = 102;
 constexpr int kLo46Per = 3;   // workgroups per CU (168 registers)
 __host__ __device__ constexpr int lo46_tile_words(int cm) { return (cm >> 6) & 1 ? 1024 : 768; }   // whole 256-word copies
@@ -698,10 +699,9 @@ __global__ __launch_bounds__(kLoThreads) __attribute__((amdgpu_waves_per_eu(3, 3
     first += w;
     if (first >= last) return;
     LoNext nx;
-    // The next tile's payload is copied into the wave's LDS buffer (direct-to-LDS loads, no registers held) before
-    // this tile's output stores, and its tile word comes through the scalar cache: stores count in vmcnt like loads,
-    // so data requested after them could only be waited for together with them. A tile's row scale and row are
-    // loaded at the start of its own iteration and first used after its decode.
+    // The next tile's payload is copied into the wave's LDS buffer (direct-to-LDS loads, no registers held) while this
+    // tile is transformed and stored; its tile word comes through the scalar cache. A tile's row scale and row are loaded
+    // at the start of its own iteration and first used after its decode.
     auto issue = [&](size_t q, int lane) {
         int g, b;
         tile_of(a, q, g, b);
@@ -720,15 +720,15 @@ __global__ __launch_bounds__(kLoThreads) __attribute__((amdgpu_waves_per_eu(3, 3
     int icb = -1;
     issue(first, lane_in);
     for (size_t q = first; q < last; q += kLoWaves) {
-        // lane-derived values formed per tile: held across the loop they would be spilled, and a spill reload waits
-        // for every memory operation in flight (this tile's stores included)
+        // lane-derived values formed per tile: held across the loop they would be spilled too
         int lane = lane_in;
         __asm__ volatile("" : "+v"(lane));
         const int j = lane & 31, p = lane >> 5, p16 = 16 * p;
         const int d = p16;
         const s16x2 sg = {(short)(p ? -1 : 1), (short)(p ? -1 : 1)};
         const int c = nx.c;
-        // this tile's copy is in LDS (the compiler does not order these reads behind the copies of lds_copy16)
+        // this tile's copy is in LDS (the compiler does not order these reads behind the copies of lds_copy16). The wait is
+        // also for the last tile's stores, which count like loads and whose number varies (rows outside the window)
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
         uint32_t w0[8], w1[8], v0[4] = {}, v1[4] = {};
         lo46_read<CM>(c, w0, pay[w], j, d);

@@ -227,7 +227,7 @@ __device__ __forceinline__ void gemv_tile_quad(const TaskCtx<NCOL, P8X_ACT_Q8_12
 // A tile whose class is known at run time only, one of the class set CM (loaded as AnyQuads): every stage's fields are
 // brought to bytes (the narrow ones; most are bytes as loaded), then one body per number of stages serves every class.
 // A body per class keeps so many registers in reach that a prefetched tile spills, and the spill reloads wait for the
-// prefetch (28 to 85 spilled registers at 128; none this way).
+// prefetch (28 to 85 spilled registers at 128 in k_gemv_rg, none this way; k_step of all classes 102 and 10).
 template <int CM>
 struct ByteFields {
     static constexpr int NST = (CM >> 7) & 1 ? 3 : (CM >> 4) & 7 ? 2 : 1;   // most stages of the set

@@ -122,6 +122,8 @@ __device__ __forceinline__ void mxs_tile(const MxsSmem<ACT> &sm, const QuadSlice
     }
 }
 
+// Spilled registers at 128: all classes 12 and 15 (q8, x16) and 2 to 12 (block_q8_1), classes 2-4 and 6 with NC 4 of q8 4,
+// class 3 with NC 2 of block_q8_1 7; the other instantiations none.
 // NC: columns a lane group holds (1, 2 or 4; 4 for more than two multiplied columns, the second group columns 4 .. 7)
 template <int ACT, int CM, int NC>
 __global__ __launch_bounds__(64 * mxs_waves()) __attribute__((amdgpu_waves_per_eu(mxs_waves() / 4, mxs_waves() / 4)))

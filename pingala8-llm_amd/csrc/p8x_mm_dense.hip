@@ -3,7 +3,8 @@
 //
 // k_mm decodes a weight tile again for every 128 or 256 tokens, and its decode (5 to 9 VALU instructions per MFMA and
 // the table reads) holds the matrix cores at about a third of their rate, less for mixed classes. Past a few hundred
-// tokens it is cheaper to write the operands v S once (2 bytes per weight) and to read them back per token tile. The
+// tokens it is cheaper to write the operands v S once (2 bytes per weight, in memory that calls share: p8x_operands.h)
+// and to read them back per token tile; a tensor with more than kMmOperandBytes goes through in bands of row tiles. The
 // operands and the order in which they are summed are k_mm's, so both give the same bits for the same K split.
 #include <hip/hip_runtime.h>
 

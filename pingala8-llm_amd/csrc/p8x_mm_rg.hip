@@ -1,4 +1,4 @@
-// p8x_mm_rg.hip -- prompt GEMM of few tokens (9 .. 64): Y [N][rows] = X [N][K] W^T in one pass over the weights.
+// p8x_mm_rg.hip -- prompt GEMM of few tokens (1 .. 64): Y [N][rows] = X [N][K] W^T in one pass over the weights.
 //
 // The products are those of p8x_gemm.hip (x' = FWHT(x ic) / 16 in fp16, weights v S rounded once to fp16, fp32 sums on
 // v_mfma_f32_32x32x16_f16); the work is split as the row-group GEMV splits it. A workgroup takes whole 32-row groups,
@@ -48,7 +48,8 @@ struct MmRgJob {
     uint32_t dbytes, sbytes;
 };
 
-// class 3 with one token tile: 16 waves at 128 VGPRs; two tiles or any class: 8 waves at 256
+// class 3 with one token tile: 16 waves at 128 VGPRs; two tiles or any class: 8 waves at 256 (any class with two tiles
+// spills 44 of them, the others none)
 __host__ __device__ constexpr int mm_rg_waves(int cm, int tt) { return cm == kMmCmC3 && tt == 1 ? 16 : 8; }
 
 // A wave's x' operands are loaded a segment of steps ahead: SEG steps x T token tiles = 8 operands, 32 registers.
