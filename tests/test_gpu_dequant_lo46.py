@@ -1,5 +1,6 @@
 """fp16 / bf16 dequantize of tensors with tiles of classes 4 and 6 beside 0-3 (integer stages up to 16 columns, then the
-reference's f32 additions; tensors of fewer tiles than CUs take the general kernel): bitwise the round-to-nearest-even of the f32 dequantize, whose bits the oracle pins."""
+reference's f32 additions; calls of fewer tiles than CUs and tensors with negative or infinite scales take the general
+kernel): bitwise the round-to-nearest-even of the f32 dequantize, whose bits the oracle pins."""
 import numpy as np
 import pytest
 
@@ -40,7 +41,8 @@ def scales(slot, rows, K):
 
 
 def test_dequant_lo46_extreme_scales():
-    """full 11-bit scale mantissas, the largest and the subnormal ones: the exactness bound's edge"""
+    """full 11-bit scale mantissas, the largest and the subnormal ones, a negative one among them, which takes the general
+    kernel (without it, the exactness bound's edge: test_dequant_lo46_extreme_positive_scales)"""
     rows, K = 1024, 2048
     slot = p8x.synth_random(5, rows, K, class_p=MIXES["c012346"], nd=6).copy()
     s = scales(slot, rows, K)
