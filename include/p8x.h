@@ -201,13 +201,14 @@ int p8x_step_create_act(const p8x_step_stage *stages, int n, int act, p8x_step *
  * clamp delta on the original X. Uses the handle's workspace (x' and output planes, N-dependent): a call with a larger N
  * than any before allocates it (synchronizing the device) unless p8x_mul_mat_reserve covered N.
  * Calls of many tokens on tensors of mixed classes decode the weights once into fp16 operands first (2 bytes per weight,
- * at most 192 MiB at a time), in a buffer that all tensors of a GPU share and that goes back with the last of them. A call
- * that does not get it (no memory, or still in use by a call on another stream) decodes as it multiplies: the same bits,
- * slower. A call that is captured in a graph allocates operands of its own instead, which stay with the tensor. */
+ * at most 192 MiB at a time), in a buffer that all tensors of a GPU share and that goes back with the last of them; calls
+ * that overlap on several streams bring up to three more. A call that gets none (no memory, or all still in use by calls on
+ * other streams) decodes as it multiplies: the same bits, slower. A call that is captured in a graph allocates operands of
+ * its own instead, which stay with the tensor. */
 int p8x_mul_mat(const p8x_tensor *t, const void *x, int x_dtype, int N, size_t ldx, float *y, size_t ldy, void *stream);
 /* No counterpart in the reference (ggml's pool allocator serves its temporaries): allocate the p8x_mul_mat
- * workspace for up to n_max tokens at set-up, so later calls with N <= n_max allocate nothing (but a captured call's
- * operands, above). Memory for the shared operands that cannot be had is no error. */
+ * workspace for up to n_max tokens at set-up, so later calls with N <= n_max allocate nothing (but the operands of captured
+ * and of overlapping calls, above). Memory for the shared operands that cannot be had is no error. */
 int p8x_mul_mat_reserve(const p8x_tensor *t, int n_max);
 /* No counterpart in the reference; for callers that cannot allocate (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc): p8x_mul_mat with its workspace (fp16 x' and K-split output planes) in a

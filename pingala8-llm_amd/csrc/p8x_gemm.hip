@@ -575,8 +575,8 @@ struct HipApi {
 
 constexpr int kMaxDevices = 64;
 struct DeviceOperands {
-    OperandBuffer<HipApi> shared;   // p8x_mul_mat
-    FixedOperands<HipApi> fixed;    // p8x_mul_mat_noalloc
+    OperandPool<HipApi> shared;    // p8x_mul_mat
+    FixedOperands<HipApi> fixed;   // p8x_mul_mat_noalloc
 };
 static DeviceOperands g_operands[kMaxDevices];
 static_assert(FixedOperands<HipApi>::kSizes[2] == kMmOperandBytes, "a band fits the largest");

@@ -38,7 +38,7 @@ struct OperandMark {
     unsigned long long *word = nullptr, n = 0;
 };
 
-// The buffer that the calls on one GPU share. One call holds it at a time (its lock spans the call's launches), and a word
+// A buffer that the calls on one GPU share. One call holds it at a time (its lock spans the call's launches), and a word
 // in host memory, which the kernel behind those that read the buffer writes, tells when the GPU is done with it. (An event
 // recorded there took 1.5 to 3 us a call, 33.0 -> 34.5 / 36.0 for 300 tokens of 1024 x 4096; given to the launch as its
 // stop event, it took 30 us of a first call after a pause.) A call on the stream that used it last is ordered behind that
@@ -125,6 +125,28 @@ private:
     typename Api::Stream last{};
     bool used = false;   // launches of the last use may still run
     int users = 0;
+};
+
+// The buffers of a GPU: one, and up to three more from when calls on as many streams have overlapped (their first use
+// allocates them). A call that finds them all in use on other streams gets none. Four, as HIP gives a process four hardware
+// queues: us a call of 4096 x 14336, classes 2-4, 1500 tokens on 1, 2 and 3 streams 199, 177 and 187 with a buffer per
+// tensor, 199, 177 and 244 with two in all.
+template <class Api>
+class OperandPool {
+public:
+    void add_user() { for (auto &x : b) x.add_user(); }
+    void drop_user() { for (auto &x : b) x.drop_user(); }
+    void reserve(size_t need) { b[0].reserve(need); }
+    typename OperandBuffer<Api>::Lease take(size_t need, typename Api::Stream st) {
+        for (auto &x : b) {
+            auto l = x.take(need, st);
+            if (l.p) return l;
+        }
+        return typename OperandBuffer<Api>::Lease();
+    }
+
+private:
+    OperandBuffer<Api> b[4];
 };
 
 // The operands of calls that may not allocate: buffers of fixed sizes, allocated when the first tensor that needs one is

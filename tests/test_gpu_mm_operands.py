@@ -82,8 +82,8 @@ def test_noalloc_decodes_first_too(rows, K, N):
     g.release()
 
 
-def test_two_streams_bitwise():
-    """three tensors' calls in turn on two streams, without waiting: whoever finds the buffer in use decodes in the GEMM"""
+def test_streams_bitwise():
+    """three tensors' calls in turn on three streams, without waiting"""
     N = 1500
     ts = [tensor(i) for i in range(3)]
     xs = [p8x.DeviceBuffer.from_numpy(np.random.default_rng(i).standard_normal((N, 4096)).astype(np.float32)) for i in range(3)]
@@ -107,26 +107,28 @@ def test_two_streams_bitwise():
 
 @pytest.mark.parametrize("rows,K,N,permute", [(4096, 4096, 1345, True), (8192, 1024, 641, False)])
 def test_busy_buffer_runs_k_mm(rows, K, N, permute):
-    """a call that finds the buffer in use on another stream (milliseconds of calls are queued there) decodes in the GEMM, on
-    the K ranges of the decoded plan: the same bits; afterwards the buffer is free for this stream too"""
+    """a call that finds every buffer in use on other streams (milliseconds of calls are queued there) decodes in the GEMM, on
+    the K ranges of the decoded plan: the same bits; afterwards a buffer is free for this stream too"""
     t = p8x.Tensor(p8x.synth_random(N, rows, K, class_p=MIX, nd=5, permute=permute), rows, K)
-    a = tensor(1)
+    others = [tensor(i) for i in range(4)]
     assert t.mul_mat_plan(N)["kernel"] == p8x.MM_DECODED
     x, xa = (p8x.DeviceBuffer.from_numpy(np.random.default_rng(i).standard_normal(s).astype(np.float32)) for i, s in enumerate(((N, K), (1500, 4096))))
-    y, ya = p8x.DeviceBuffer(4 * N * rows), p8x.DeviceBuffer(4 * 1500 * 4096)
+    y, ys = p8x.DeviceBuffer(4 * N * rows), [p8x.DeviceBuffer(4 * 1500 * 4096) for _ in others]
     t.mul_mat_reserve(N)
-    a.mul_mat_reserve(1500)
+    for a in others:
+        a.mul_mat_reserve(1500)
     t.mul_mat_dev(x, p8x.F32, N, y)
     p8x.synchronize()
     ref = y.to_numpy(np.uint32, (N, rows)).copy()
-    s1, s2 = p8x.Stream(), p8x.Stream()
+    st, sts = p8x.Stream(), [p8x.Stream() for _ in others]
     for busy in (True, False):
         y.fill(0xFF)
         p8x.synchronize()
         if busy:
-            for _ in range(60):
-                a.mul_mat_dev(xa, p8x.F32, 1500, ya, stream=s1)
-        t.mul_mat_dev(x, p8x.F32, N, y, stream=s2)
+            for _ in range(30):
+                for a, ya, s in zip(others, ys, sts):
+                    a.mul_mat_dev(xa, p8x.F32, 1500, ya, stream=s)
+        t.mul_mat_dev(x, p8x.F32, N, y, stream=st)
         p8x.synchronize()
         assert np.array_equal(y.to_numpy(np.uint32, (N, rows)), ref)
 

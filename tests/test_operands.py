@@ -17,8 +17,8 @@ FAKE = r"""
 struct Fake {   // log: a = alloc, f = free, s = device synchronize, c = error cleared
     using Stream = int;
     static bool cap;   // streams are being captured
-    static unsigned long long *word;
-    static bool host_word(unsigned long long **p) { static unsigned long long w; word = *p = &w; return true; }
+    static unsigned long long *word;   // of the buffer that asked last
+    static bool host_word(unsigned long long **p) { word = *p = new unsigned long long(0); return true; }
     static bool ordered(Stream a, Stream b) { return a == b && a != 0; }
     static bool capturing(Stream) { return cap; }
     static std::string log;
@@ -184,4 +184,29 @@ def test_fixed_operands(tmp_path):
     assert(f.get(M) == p && Fake::held == 80 * M);   // a captured call may hold either
     f.drop_user();
     assert(!f.get(M) && Fake::held == 0);
+    """)
+
+
+def test_pool(tmp_path):
+    """a further buffer for each stream that overlaps, none for a fifth; all go back with the last user"""
+    run(tmp_path, r"""
+    OperandPool<Fake> pool;
+    Fake::room = 1000;
+    pool.add_user();
+    pool.reserve(100);
+    assert(Fake::held == 100);
+    void *p[5];
+    for (int round = 0; round < 2; ++round)
+        for (int st = 1; st <= 5; ++st) {
+            auto l = pool.take(100, st);
+            if (l.p) l.launched();
+            if (round == 0) {
+                p[st - 1] = l.p;
+                for (int i = 0; i < st - 1; ++i) assert(l.p != p[i]);
+            }
+            assert(l.p == p[st - 1] && Fake::held == 100u * (round ? 4 : st < 5 ? st : 4));
+        }
+    assert(p[3] && !p[4]);
+    pool.drop_user();
+    assert(Fake::held == 0);
     """)
